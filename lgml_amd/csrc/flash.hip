@@ -4,10 +4,32 @@
 // It serves callers whose K / V are plain (n_kv, Hkv * D) rows rather than
 // this library's block pool (the paged path is attn.hip).
 //
-// One wave64 per (query row, head). Per tile of 64 columns each lane
-// scores one column (q from LDS against its own K row, 16-byte loads), the
-// wave takes the tile max and sum with shuffles (online softmax in f32),
-// and each lane accumulates D / 64 output values from coalesced V rows.
+// The rows of a KV head are its T * G (token, query head) pairs, 16 to a
+// wave. A workgroup is KW groups of RW waves: the waves of a group take
+// consecutive row tiles over the same cells, the groups take the 64- (or 32-)
+// cell tiles in turn (tile i is group i % KW's), and their states are merged
+// in group order at the end. Per tile a group stages K as rows and V
+// transposed in LDS, from registers that were loaded while the tile before
+// was computed; a wave computes S^T = K Q^T with 16x16x32 f16 MFMAs, an
+// online softmax in f32 (a lane owns one row), and O^T += V^T P^T.
+//
+// K and V are exact f16; Q (scaled by a power of two to at most 1 per row,
+// so any f32 row fits f16) and P enter the MFMAs as f16 hi + lo pairs, so a
+// product is f32-accurate. The MFMA's k index over 32 cells is taken in the
+// order (quad, tile of 16, i): a lane's own S^T values then are its B operand
+// of the second product, with no trip through LDS, and V^T is stored in that
+// order of cells.
+//
+// A masked cell (mask -inf, or past n_kv) adds nothing whatever K and V
+// hold there: its score is set, and a V value that is not finite is stored
+// as 0 for the MFMAs and added afterwards to the rows that do see its cell.
+//
+// What bounds it: the f16 MFMAs (twice the products' flops for the hi + lo
+// pairs) and the softmax's VALU, which overlap only in part (the two waves of
+// a SIMD run in step). 32 / 8 heads of 128, 512 rows over 2048 cells under a
+// causal mask: 72.7 us, 207 TFLOP/s of the products (2460 us with one wave
+// per query row and head, each column's dot product in VALU); without its
+// loads 56 us, without its products and softmax 27.
 #include <math.h>
 
 #include "common.h"
@@ -15,15 +37,7 @@
 namespace lgmlh {
 
 constexpr int FA_MAX_D = 256;
-
-__device__ __forceinline__ float wave_max(float v) {
-  for (int o = 32; o > 0; o >>= 1) v = fmaxf(v, __shfl_xor(v, o));
-  return v;
-}
-__device__ __forceinline__ float wave_sum(float v) {
-  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o);
-  return v;
-}
+constexpr float FA_LOG2E = 1.4426950408889634f;
 
 // ALiBi slope of head h (1 without max_bias): with n the largest power of
 // two <= H, heads below n take (2^(-max_bias / n))^(h + 1), the others
@@ -37,71 +51,503 @@ __device__ __forceinline__ float alibi(int h, int H, float max_bias) {
   return h < n ? powf(m0, (float)(h + 1)) : powf(m1, (float)(2 * (h - n) + 1));
 }
 
-__global__ void __launch_bounds__(64)
-flash_attn_kernel(const float *__restrict__ q, int H, int T, int D,
-                  const uint16_t *__restrict__ k, const uint16_t *__restrict__ v, int G, int n_kv,
-                  int64_t k_rs, int64_t k_hs, int64_t v_rs, int64_t v_hs,
-                  const uint16_t *__restrict__ mask, int mask_heads, int mask_rows, float scale,
-                  float max_bias, float softcap, float *__restrict__ out) {
-  __shared__ float qs[FA_MAX_D];
-  const int t = blockIdx.x, h = blockIdx.y, lane = threadIdx.x;
-  const int kh = h / G;
-  const float *qr = q + ((int64_t)h * T + t) * D;
-  for (int i = lane; i < D; i += 64) qs[i] = qr[i];
-  __syncthreads();
-  const uint16_t *mr = mask ? mask + ((int64_t)(h % mask_heads) * mask_rows + t) * n_kv : nullptr;
-  const float slope = alibi(h, H, max_bias);
+// Vectors of memory that need not be aligned to their size (Q, V, mask and
+// out start anywhere their elements may; the hardware loads such addresses,
+// and aligned ones as fast as ever).
+typedef float f32x2 __attribute__((ext_vector_type(2)));
+typedef f32x4 f32x4_u __attribute__((aligned(4)));
+typedef u32x4 u32x4_u __attribute__((aligned(2)));
+typedef u32x2 u32x2_u __attribute__((aligned(2)));
+
+struct FlashArgs {
+  const float *q;
+  const uint16_t *k, *v, *mask;
+  float *out;
+  int H, T, D, G, n_kv, mask_heads, mask_rows;
+  int64_t k_rs, k_hs, v_rs, v_hs;
+  float scale, max_bias, softcap;
+};
+
+// A workgroup barrier that waits for LDS operations only: global loads stay
+// in flight across it.
+__device__ __forceinline__ void fa_barrier() {
+  __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0)
+  asm volatile("" ::: "memory");
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
+}
+
+// DP: the head size padded to the MFMA step (zeros past D); BC: cells per
+// tile.
+template <int DP, int BC, int RW, int KW>
+__global__ void __launch_bounds__(RW *KW * 64, 1) flash_attn_kernel(FlashArgs A) {
+  constexpr int KS = DP / 32, DT = DP / 16, CT = BC / 16, CJ = BC / 32;
+  constexpr int KROW = DP + 8, VROW = BC + 8;  // f16 per LDS row: conflict-free 16-row reads
+  // A group of one wave takes its K fragments straight from memory.
+  constexpr bool KLDS = RW > 1;
+  constexpr int KT = KLDS ? BC * KROW : 0, VT = DP * VROW, NT = RW * 64;
+  constexpr int KU = (BC * (DP / 8) + NT - 1) / NT;        // 16-byte K pieces per thread
+  constexpr int VU = ((BC / 4) * (DP / 8) + NT - 1) / NT;  // V pieces of 4 cells x 8 values
+  constexpr int NB = KLDS ? 2 : 1;                         // stages
+  constexpr int STAGE = NB * KW * (KT + VT) * 2;           // bytes
+  constexpr int STATE = KW > 1 ? KW * RW * 16 * (DP + 2) * 4 : 0;
+  __shared__ __align__(16) uint8_t lds[STAGE > STATE ? STAGE : STATE];
+  __shared__ uint32_t bad[3][KW][2];  // cells of a tile with a V value that is not finite
+
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int kw = wave / RW, rw = wave % RW;
+  const int gt = threadIdx.x - kw * NT;  // thread of the group
+  uint16_t *const stage0 = (uint16_t *)lds + kw * NB * (KT + VT);
+  auto kl_of = [&](int it) { return stage0 + (NB == 2 ? (it & 1) * (KT + VT) : 0); };
+  const int D = A.D, kvh = blockIdx.x;
+  const int r16 = lane & 15, quad = lane >> 4;
+  const int rows = A.T * A.G;
+  const int rr = (blockIdx.y * RW + rw) * 16 + r16;
+  const bool rvalid = rr < rows;
+  const int t = (rvalid ? rr : 0) / A.G, h = kvh * A.G + (rvalid ? rr : 0) % A.G;
+  const float slope = alibi(h, A.H, A.max_bias);
+  const uint16_t *mr = A.mask ? A.mask + ((int64_t)(h % A.mask_heads) * A.mask_rows + t) * A.n_kv
+                              : nullptr;
+  const uint16_t *kb = A.k + (int64_t)kvh * A.k_hs, *vb = A.v + (int64_t)kvh * A.v_hs;
+  const int ntiles = (A.n_kv + BC - 1) / BC;
+
+  if (threadIdx.x < 6 * KW) (&bad[0][0][0])[threadIdx.x] = 0;
+
+  // Q fragments: row rr scaled by 2^-e (e the exponent of its largest |q|),
+  // hi + lo.
+  f16x8 qh[KS], ql[KS];
+  float qscale = 1.0f;
+  {
+    const float *qr = A.q + ((int64_t)h * A.T + t) * D;
+    float x[KS][8], mx = 0.0f;
+#pragma unroll
+    for (int ks = 0; ks < KS; ks++) {
+      const int d0 = ks * 32 + quad * 8;
+      f32x4 a = {0, 0, 0, 0}, b = a;
+      if (d0 < D && rvalid) {
+        a = *(const f32x4_u *)(qr + d0);
+        b = *(const f32x4_u *)(qr + d0 + 4);
+      }
+#pragma unroll
+      for (int e = 0; e < 4; e++) {
+        x[ks][e] = a[e];
+        x[ks][4 + e] = b[e];
+      }
+#pragma unroll
+      for (int e = 0; e < 8; e++) mx = fmaxf(mx, fabsf(x[ks][e]));
+    }
+    mx = fmaxf(mx, __shfl_xor(mx, 16));
+    mx = fmaxf(mx, __shfl_xor(mx, 32));
+    // exponents of f32 normals; a zero, denormal or infinite maximum keeps 1
+    const int ex = (int)(__builtin_bit_cast(uint32_t, mx) >> 23);
+    float inv = 1.0f;
+    if (ex > 1 && ex < 253) {
+      inv = __builtin_bit_cast(float, (uint32_t)(253 - ex) << 23);
+      qscale = __builtin_bit_cast(float, (uint32_t)(ex + 1) << 23);
+    }
+#pragma unroll
+    for (int ks = 0; ks < KS; ks++)
+#pragma unroll
+      for (int e = 0; e < 8; e++) {
+        const float v = x[ks][e] * inv;
+        qh[ks][e] = (f16)v;
+        ql[ks][e] = (f16)(v - (float)qh[ks][e]);
+      }
+  }
   // with a softcap the scale goes inside the tanh: softcap tanh(s (scale / softcap))
-  const float sc = softcap > 0.0f ? scale / softcap : scale;
-  const uint16_t *kb = k + (int64_t)kh * k_hs, *vb = v + (int64_t)kh * v_hs;
-  float m = -INFINITY, l = 0.0f, o[FA_MAX_D / 64];
+  const float sc = (A.softcap > 0.0f ? A.scale / A.softcap : A.scale) * qscale;
+
+  // A tile's K rows, V pieces and mask values in registers. Cells past n_kv
+  // repeat the last one and are masked. In whole tiles a thread's rows are
+  // fixed distances from its first, so that its addresses take one add each.
+  u32x4 kr[KU], vr[VU][4];
+  u32x2 mk[CT];  // 4 cells of f16 bits (taken apart only when they are used)
+  constexpr bool KSTEP = !KLDS || NT % (DP / 8) == 0;
+  static_assert(NT % (BC / 4) == 0, "a thread's V pieces are of the same cells");
+  auto k_row = [&](int u) { return KLDS ? (gt + u * NT) / (DP / 8) : u / KS * 16 + r16; };
+  auto k_col = [&](int u) { return KLDS ? (gt + u * NT) % (DP / 8) * 8 : u % KS * 32 + quad * 8; };
+  const int vc0 = gt % (BC / 4) * 4;
+  auto v_col = [&](int u) { return (gt + u * NT) / (BC / 4) * 8; };
+  const uint16_t *const kp0 = kb + (int64_t)k_row(0) * A.k_rs + k_col(0);
+  const uint16_t *const vp0 = vb + (int64_t)vc0 * A.v_rs + v_col(0);
+  auto load_k = [&](int tile) {
+    const int j0 = tile * BC, jl = A.n_kv - 1;
+    if (KSTEP && D == DP && j0 + BC <= A.n_kv) {
+      const uint16_t *p = kp0 + (int64_t)j0 * A.k_rs;
 #pragma unroll
-  for (int i = 0; i < FA_MAX_D / 64; i++) o[i] = 0.0f;
-  for (int j0 = 0; j0 < n_kv; j0 += 64) {
-    const int j = j0 + lane;
-    float s = -INFINITY;
-    if (j < n_kv) {
-      const float mv = mr ? h2f(mr[j]) : 0.0f;
-      if (mv != -INFINITY) {
-        const uint16_t *kr = kb + (int64_t)j * k_rs;
-        float a = 0.0f;
-        for (int d = 0; d < D; d += 8) {
-          const u32x4 w = *(const u32x4 *)(kr + d);
+      for (int u = 0; u < KU; u++)
+        kr[u] = KLDS ? *(const u32x4 *)(p + (int64_t)(u * (NT / (DP / 8))) * A.k_rs)
+                     : *(const u32x4 *)(p + (int64_t)(u / KS * 16) * A.k_rs + u % KS * 32);
+      return;
+    }
 #pragma unroll
-          for (int e = 0; e < 4; e++) {
-            a = fmaf(qs[d + 2 * e], h2f((uint16_t)(w[e] & 0xffffu)), a);
-            a = fmaf(qs[d + 2 * e + 1], h2f((uint16_t)(w[e] >> 16)), a);
-          }
-        }
-        a *= sc;
-        if (softcap > 0.0f) a = softcap * tanhf(a);
-        s = a + slope * mv;
+    for (int u = 0; u < KU; u++) {
+      const int d0 = k_col(u);
+      kr[u] = *(const u32x4 *)(kb + (int64_t)min(j0 + k_row(u), jl) * A.k_rs + (d0 < D ? d0 : 0));
+      if (d0 >= D) kr[u] = u32x4{0, 0, 0, 0};
+    }
+  };
+  auto load_vm = [&](int tile) {
+    const int j0 = tile * BC, jl = A.n_kv - 1;
+    if (D == DP && VU * NT == BC / 4 * (DP / 8) && j0 + BC <= A.n_kv) {
+      const uint16_t *p = vp0 + (int64_t)j0 * A.v_rs;
+#pragma unroll
+      for (int u = 0; u < VU; u++)
+#pragma unroll
+        for (int i = 0; i < 4; i++)
+          vr[u][i] = *(const u32x4_u *)(p + i * A.v_rs + u * (NT / (BC / 4)) * 8);
+    } else {
+#pragma unroll
+      for (int u = 0; u < VU; u++) {
+        const uint16_t *s = vb + (v_col(u) < D ? v_col(u) : 0);
+#pragma unroll
+        for (int i = 0; i < 4; i++)
+          vr[u][i] = *(const u32x4_u *)(s + (int64_t)min(j0 + vc0 + i, jl) * A.v_rs);
       }
     }
-    const float mt = wave_max(s);
-    if (mt == -INFINITY) continue;  // every column of the tile is masked
-    const float mn = fmaxf(m, mt);
-    const float corr = expf(m - mn);  // 0 while m is -inf
-    const float p = s == -INFINITY ? 0.0f : expf(s - mn);
-    l = l * corr + wave_sum(p);
+    if (mr && j0 + BC <= A.n_kv) {
 #pragma unroll
-    for (int i = 0; i < FA_MAX_D / 64; i++) o[i] *= corr;
-    const int nj = n_kv - j0 < 64 ? n_kv - j0 : 64;
-    for (int jj = 0; jj < nj; jj++) {
-      const float pj = __shfl(p, jj);
-      if (pj == 0.0f) continue;  // wave-uniform
-      const uint16_t *vr = vb + (int64_t)(j0 + jj) * v_rs;
+      for (int ct = 0; ct < CT; ct++) mk[ct] = *(const u32x2_u *)(mr + j0 + ct * 16 + quad * 4);
+    } else {
 #pragma unroll
-      for (int i = 0; i < FA_MAX_D / 64; i++)
-        if (lane + 64 * i < D) o[i] = fmaf(pj, h2f(vr[lane + 64 * i]), o[i]);
+      for (int ct = 0; ct < CT; ct++) {
+        uint32_t b[4];
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+          const int j = j0 + ct * 16 + quad * 4 + i;
+          b[i] = j > jl ? 0xfc00u : mr ? mr[min(j, jl)] : 0u;
+        }
+        mk[ct] = u32x2{b[0] | (b[1] << 16), b[2] | (b[3] << 16)};
+      }
     }
-    m = mn;
-  }
-  float *orow = out + ((int64_t)t * H + h) * D;
-  const float inv = l > 0.0f ? 1.0f / l : 0.0f;
+  };
+  // The registers of a tile to LDS: K rows, V transposed (4 cells of a value
+  // are 8 bytes).
+  auto store = [&](int it) {
+    uint16_t *const kl = kl_of(it), *const vl = kl + KT;
+    if constexpr (KLDS) {
 #pragma unroll
-  for (int i = 0; i < FA_MAX_D / 64; i++)
-    if (lane + 64 * i < D) orow[lane + 64 * i] = o[i] * inv;
+      for (int u = 0; u < KU; u++) {
+        if (k_row(u) < BC) *(u32x4 *)(kl + k_row(u) * KROW + k_col(u)) = kr[u];
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < VU; u++) {
+      const int c0 = vc0, d0 = v_col(u);
+      uint32_t nf = 0;  // bits 15, 31: an exponent of all ones
+#pragma unroll
+      for (int i = 0; i < 4; i++)
+#pragma unroll
+        for (int e = 0; e < 4; e++) nf |= (vr[u][i][e] & 0x7fff7fffu) + 0x04000400u;
+      if (__builtin_expect((nf & 0x80008000u) != 0, 0)) {
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+          bool any = false;
+#pragma unroll
+          for (int e = 0; e < 4; e++) {
+            const uint32_t w = vr[u][i][e], f = ((w & 0x7fff7fffu) + 0x04000400u) & 0x80008000u;
+            any = any || f;
+            vr[u][i][e] = w & ~((f >> 15) * 0xffffu);
+          }
+          if (any) atomicOr(&bad[it % 3][kw][(c0 + i) >> 5], 1u << ((c0 + i) & 31));
+        }
+      }
+      // cell c of a tile of 32 at place (c % 16 / 4) * 8 + c / 16 * 4 + c % 4
+      const int place = (c0 & ~31) + ((c0 & 15) >> 2) * 8 + ((c0 >> 4) & 1) * 4;
+      if (d0 < DP)
+#pragma unroll
+        for (int e = 0; e < 8; e++) {
+          const uint32_t s = (e & 1) ? 0x07060302u : 0x05040100u;
+          const u32x2 w = {__builtin_amdgcn_perm(vr[u][1][e >> 1], vr[u][0][e >> 1], s),
+                           __builtin_amdgcn_perm(vr[u][3][e >> 1], vr[u][2][e >> 1], s)};
+          *(u32x2 *)(vl + (d0 + e) * VROW + place) = w;
+        }
+    }
+  };
+
+  f32x4 o[DT];
+#pragma unroll
+  for (int i = 0; i < DT; i++) o[i] = f32x4{0, 0, 0, 0};
+  float m = -INFINITY, l = 0.0f;
+
+  // S^T of a tile.
+  f32x4 st[CT];
+  auto scores = [&](const uint16_t *kl) {
+    // K fragments of a step over D are read while the one before multiplies
+    f16x8 kf[2][CT];
+    auto read = [&](int ks, f16x8(&f)[CT]) {
+#pragma unroll
+      for (int ct = 0; ct < CT; ct++)
+        f[ct] = KLDS ? *(const f16x8 *)(kl + (ct * 16 + r16) * KROW + ks * 32 + quad * 8)
+                     : __builtin_bit_cast(f16x8, kr[(ct * KS + ks) % KU]);
+    };
+    read(0, kf[0]);
+#pragma unroll
+    for (int ks = 0; ks < KS; ks++) {
+      if (ks + 1 < KS) read(ks + 1, kf[(ks + 1) & 1]);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int ct = 0; ct < CT; ct++)
+        st[ct] = __builtin_amdgcn_mfma_f32_16x16x32_f16(
+            kf[ks & 1][ct], qh[ks], ks ? st[ct] : f32x4{0, 0, 0, 0}, 0, 0, 0);
+#pragma unroll
+      for (int ct = 0; ct < CT; ct++)
+        st[ct] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kf[ks & 1][ct], ql[ks], st[ct], 0, 0, 0);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  };
+  // The softmax of a tile (its mask values in mc) and its products with V.
+  auto compute = [&](int tile, int it, const uint16_t *vl, const u32x2 (&mc)[CT]) {
+#pragma unroll
+    for (int ct = 0; ct < CT; ct++) st[ct] *= sc;
+    if (A.softcap > 0.0f) {
+#pragma unroll 1
+      for (int ct = 0; ct < CT; ct++) {
+        f32x4 x = st[0];
+#pragma unroll
+        for (int i = 0; i < 4; i++) x[i] = A.softcap * tanhf(x[i]);
+        // the tiles rotate through st[0], so that no register is indexed
+#pragma unroll
+        for (int c2 = 0; c2 + 1 < CT; c2++) st[c2] = st[c2 + 1];
+        st[CT - 1] = x;
+      }
+    }
+    uint32_t any = 0;
+#pragma unroll
+    for (int ct = 0; ct < CT; ct++) any |= mc[ct][0] | mc[ct][1];
+    if (__builtin_amdgcn_ballot_w64(any != 0)) {  // else every mask value of the tile is 0
+#pragma unroll
+      for (int ct = 0; ct < CT; ct++)
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+          const float b = h2f((uint16_t)(mc[ct][i >> 1] >> (16 * (i & 1))));
+          st[ct][i] = b == -INFINITY ? -INFINITY : st[ct][i] + slope * b;
+        }
+    }
+    float mx = -INFINITY;
+#pragma unroll
+    for (int ct = 0; ct < CT; ct++)
+#pragma unroll
+      for (int i = 0; i < 4; i++) mx = fmaxf(mx, st[ct][i]);
+    mx = fmaxf(mx, __shfl_xor(mx, 16));
+    mx = fmaxf(mx, __shfl_xor(mx, 32));
+    const float m_new = fmaxf(m, mx);
+    const float m_use = m_new == -INFINITY ? 0.0f : m_new;
+    float rs = 0.0f;
+#pragma unroll
+    for (int ct = 0; ct < CT; ct++)
+#pragma unroll
+      for (int i = 0; i < 4; i++) {
+        st[ct][i] = __builtin_amdgcn_exp2f((st[ct][i] - m_use) * FA_LOG2E);  // exp2(-inf) = 0
+        rs += st[ct][i];
+      }
+    rs += __shfl_xor(rs, 16);
+    rs += __shfl_xor(rs, 32);
+    if (__builtin_amdgcn_ballot_w64(m_new != m)) {
+      const float alpha = __builtin_amdgcn_exp2f((m - m_use) * FA_LOG2E);  // 0 while m is -inf
+      l *= alpha;
+#pragma unroll
+      for (int dt = 0; dt < DT; dt++) o[dt] *= alpha;
+    }
+    l += rs;
+    m = m_new;
+    f16x8 ph[CJ], pl[CJ];
+#pragma unroll
+    for (int j = 0; j < CJ; j++)
+#pragma unroll
+      for (int e = 0; e < 8; e += 2) {
+        const f32x2 p = {st[2 * j + (e >> 2)][e & 3], st[2 * j + (e >> 2)][(e & 3) + 1]};
+        const f16x2 hi = __builtin_convertvector(p, f16x2);
+        const f32x2 r = {fmaf((float)hi[0], -1.0f, p[0]), fmaf((float)hi[1], -1.0f, p[1])};
+        const f16x2 lo = __builtin_convertvector(r, f16x2);
+        ph[j][e] = hi[0];
+        ph[j][e + 1] = hi[1];
+        pl[j][e] = lo[0];
+        pl[j][e + 1] = lo[1];
+      }
+    f16x8 vf[2][CJ];
+    auto read = [&](int dt, f16x8(&f)[CJ]) {
+#pragma unroll
+      for (int j = 0; j < CJ; j++)
+        f[j] = *(const f16x8 *)(vl + (dt * 16 + r16) * VROW + j * 32 + quad * 8);
+    };
+    // two tiles of D at a time, the next two read meanwhile
+    static_assert(DT % 2 == 0, "d tiles in pairs");
+    f16x8 vg[2][CJ];
+    read(0, vf[0]);
+    read(1, vg[0]);
+#pragma unroll
+    for (int dt = 0; dt < DT; dt += 2) {
+      const int b = dt >> 1 & 1;
+      if (dt + 2 < DT) {
+        read(dt + 2, vf[b ^ 1]);
+        read(dt + 3, vg[b ^ 1]);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int j = 0; j < CJ; j++) {
+        o[dt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vf[b][j], ph[j], o[dt], 0, 0, 0);
+        o[dt + 1] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vg[b][j], ph[j], o[dt + 1], 0, 0, 0);
+        o[dt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vf[b][j], pl[j], o[dt], 0, 0, 0);
+        o[dt + 1] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vg[b][j], pl[j], o[dt + 1], 0, 0, 0);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    // V values that are not finite, to the rows that see their cells
+    for (int w = 0; w < 2; w++) {
+      uint32_t b = __builtin_amdgcn_readfirstlane(bad[it % 3][kw][w]);
+      for (; b; b &= b - 1) {
+        const int c = 32 * w + __builtin_ctz(b);
+        float p = 0.0f;
+#pragma unroll
+        for (int ct = 0; ct < CT; ct++)
+#pragma unroll
+          for (int i = 0; i < 4; i++)
+            if (c == ct * 16 + (c & 12) + i) p = st[ct][i];
+        p = __shfl(p, ((c & 12) >> 2) * 16 + r16);
+        const uint16_t *vs = vb + (int64_t)min(tile * BC + c, A.n_kv - 1) * A.v_rs;
+#pragma unroll
+        for (int dt = 0; dt < DT; dt++)
+#pragma unroll
+          for (int i = 0; i < 4; i++) {
+            const int d = dt * 16 + quad * 4 + i;
+            const uint16_t x = d < D ? vs[d] : 0;
+            if (p != 0.0f && (x & 0x7c00) == 0x7c00) o[dt][i] += p * h2f(x);
+          }
+      }
+    }
+  };
+
+  // Tile it * KW + kw: its registers go to LDS, the next tile's loads go out,
+  // then it is computed. All groups take the same number of turns. A group of
+  // one wave needs no barrier: its LDS operations complete in order.
+  auto turn_barrier = [&]() {
+    if constexpr (KLDS)
+      fa_barrier();
+    else
+      asm volatile("" ::: "memory");
+  };
+  // Loads are unconditional: tiles past the last repeat its last cell, all
+  // masked. With two stages a tile is computed from one while the next
+  // tile's registers, loaded meanwhile, wait for the other: one barrier a
+  // turn.
+  const int turns = (ntiles + KW - 1) / KW;
+  fa_barrier();  // bad starts at zero
+  u32x2 mc[CT];
+  auto take_mask = [&]() {
+#pragma unroll
+    for (int ct = 0; ct < CT; ct++) mc[ct] = mk[ct];
+  };
+  if (turns > 0) {
+    load_k(kw);
+    load_vm(kw);
+    if constexpr (KLDS) {
+      store(0);
+      take_mask();
+      load_k(KW + kw);
+      load_vm(KW + kw);
+    }
+  }
+  for (int it = 0; it < turns; it++) {
+    const int tile = it * KW + kw;
+    turn_barrier();
+    if constexpr (!KLDS) {
+      store(it);
+      take_mask();
+      load_vm(tile + KW);
+      turn_barrier();
+    }
+    if (gt < 2) bad[(it + 2) % 3][kw][gt] = 0;  // read last in the turn before
+    const uint16_t *const kl = kl_of(it), *const vl = kl + KT;
+    bool seen = false;
+#pragma unroll
+    for (int ct = 0; ct < CT; ct++)
+      seen = seen || mc[ct][0] != 0xfc00fc00u || mc[ct][1] != 0xfc00fc00u;
+    // a tile that no row of the wave sees adds nothing
+    const bool some = __builtin_amdgcn_ballot_w64(seen && rvalid) != 0;
+    if (!KLDS || some) scores(kl);
+    if constexpr (!KLDS) load_k(tile + KW);
+    if (some) compute(tile, it, vl, mc);
+    if constexpr (KLDS) {
+      store(it + 1);
+      take_mask();
+      load_k(tile + 2 * KW);
+      load_vm(tile + 2 * KW);
+    }
+  }
+
+  if constexpr (KW > 1) {
+    // the groups' states of a row tile, merged in group order
+    float *const sl = (float *)lds;
+    auto state = [&](int g) { return sl + (g * RW + rw) * 16 * (DP + 2); };
+    fa_barrier();
+    {
+      float *s = state(kw);
+#pragma unroll
+      for (int dt = 0; dt < DT; dt++) *(f32x4 *)(s + (dt * 64 + lane) * 4) = o[dt];
+      if (quad == 0) {
+        s[16 * DP + r16] = m;
+        s[16 * DP + 16 + r16] = l;
+      }
+    }
+    fa_barrier();
+    if (kw != 0) return;
+    float M = -INFINITY;
+#pragma unroll
+    for (int g = 0; g < KW; g++) M = fmaxf(M, state(g)[16 * DP + r16]);
+    const float mu = M == -INFINITY ? 0.0f : M;
+    l = 0.0f;
+#pragma unroll
+    for (int dt = 0; dt < DT; dt++) o[dt] = f32x4{0, 0, 0, 0};
+#pragma unroll
+    for (int g = 0; g < KW; g++) {
+      const float *s = state(g);
+      const float w = __builtin_amdgcn_exp2f((s[16 * DP + r16] - mu) * FA_LOG2E);
+      l += s[16 * DP + 16 + r16] * w;
+#pragma unroll
+      for (int dt = 0; dt < DT; dt++) o[dt] += *(const f32x4 *)(s + (dt * 64 + lane) * 4) * w;
+    }
+  }
+  if (!rvalid) return;
+  // a row with every cell masked gives zeros
+  const float inv = l == 0.0f ? 0.0f : 1.0f / l;
+  float *orow = A.out + ((int64_t)t * A.H + h) * D;
+#pragma unroll
+  for (int dt = 0; dt < DT; dt++) {
+    const int d0 = dt * 16 + quad * 4;
+    if (d0 >= D) continue;
+    *(f32x4_u *)(orow + d0) = o[dt] * inv;
+  }
+}
+
+template <int DP, int BC, int RW, int KW>
+static void launch_flash(const FlashArgs &A, int n_head_kv, hipStream_t st) {
+  const int64_t rows = (int64_t)A.T * A.G;
+  hipLaunchKernelGGL((flash_attn_kernel<DP, BC, RW, KW>),
+                     dim3((unsigned)n_head_kv, (unsigned)((rows + RW * 16 - 1) / (RW * 16))),
+                     dim3(RW * KW * 64), 0, st, A);
+}
+
+// The split of a call: RW row tiles of 16 share a workgroup's K and V, KW
+// groups share its cells. From 96 workgroups of 64 rows up, four row tiles
+// (one wave per SIMD and group) in two groups (one past 128, whose stages
+// fill LDS). Below, most CUs would stay idle: one row tile per workgroup,
+// its cells over 8 waves (4 past 128, whose registers take a SIMD each),
+// K straight from memory. (32 / 8 heads of 128, 2048 cells: 200 rows, 104
+// workgroups of 64 rows, 64.6 us; 100 rows as 16-row workgroups 40.7; one
+// row 36.4, 670 in the wave-per-row kernel before.) A single 32-cell tile
+// needs one wave: nothing to merge.
+template <int DP>
+static void flash_for(const FlashArgs &A, int n_head_kv, hipStream_t st) {
+  const int64_t tiles = ((int64_t)A.T * A.G + 63) / 64 * n_head_kv;
+  constexpr int WIDE = DP <= 128 ? 2 : 1, SPLIT = DP <= 128 ? 8 : 4;
+  if (tiles >= 96)
+    launch_flash<DP, 64, 4, WIDE>(A, n_head_kv, st);
+  else if (A.n_kv > 32)
+    launch_flash<DP, 32, 1, SPLIT>(A, n_head_kv, st);
+  else
+    launch_flash<DP, 32, 1, 1>(A, n_head_kv, st);
 }
 
 }  // namespace lgmlh
@@ -131,9 +577,21 @@ extern "C" int lgmlh_flash_attn(const float *q, int n_head, int n_tokens, int he
     return LGMLH_EINVAL;
   }
   if (n_tokens == 0) return LGMLH_OK;
-  hipLaunchKernelGGL(flash_attn_kernel, dim3((unsigned)n_tokens, (unsigned)n_head), dim3(64), 0,
-                     as_stream(stream), q, n_head, n_tokens, head_dim, k, v, n_head / n_head_kv,
-                     n_kv, k_row_stride, k_head_stride, v_row_stride, v_head_stride, mask,
-                     mask_heads, mask_rows, scale, max_bias, softcap, out);
+  const FlashArgs A{q, k, v, mask, out, n_head, n_tokens, head_dim, n_head / n_head_kv, n_kv,
+                    mask ? mask_heads : 1, mask_rows, k_row_stride, k_head_stride, v_row_stride,
+                    v_head_stride, scale, max_bias, softcap};
+  hipStream_t st = as_stream(stream);
+  if (head_dim <= 32)
+    flash_for<32>(A, n_head_kv, st);
+  else if (head_dim <= 64)
+    flash_for<64>(A, n_head_kv, st);
+  else if (head_dim <= 96)
+    flash_for<96>(A, n_head_kv, st);
+  else if (head_dim <= 128)
+    flash_for<128>(A, n_head_kv, st);
+  else if (head_dim <= 192)
+    flash_for<192>(A, n_head_kv, st);
+  else
+    flash_for<256>(A, n_head_kv, st);
   return hip_check(hipGetLastError(), "flash_attn");
 }

@@ -134,3 +134,90 @@ def test_flash_attn_on_pool_rows_equals_paged_attention(L):
                         1.0 / np.sqrt(D))
         assert rel_err(got.reshape(n * H, D), paged[off:off + n].reshape(n * H, D)) < 1e-5, i
         off += n
+
+
+# Edges of the kernel's tiles: cells around 32 and 64 and the groups that
+# share them, rows around 16 and 64 (the last two cases: from 96 workgroups
+# of 64 rows, four row tiles each), head sizes that are and are not whole
+# MFMA steps. The bound is the one of the other cases: hi + lo pairs carry 22
+# bits, so products and their f32 sums over up to 256 + 300 terms stay within
+# 556 * 2^-24 + 2^-21 of the largest term, 3.4e-5; errors add at random and
+# measure 4e-7.
+EDGES = [  # H, Hkv, T, D, n_kv
+    (1, 1, 1, 8, 1), (3, 1, 5, 16, 31), (2, 2, 16, 40, 32), (4, 1, 4, 64, 33), (4, 2, 9, 96, 63),
+    (2, 1, 8, 128, 64), (8, 2, 1, 128, 65), (2, 1, 3, 160, 129), (2, 2, 17, 192, 255),
+    (8, 1, 2, 256, 257), (32, 32, 129, 72, 130), (16, 8, 395, 128, 70), (8, 8, 800, 256, 40),
+]
+
+
+@pytest.mark.parametrize("case", range(len(EDGES)))
+def test_flash_attn_tile_edges(L, case):
+    H, Hkv, T, D, n_kv = EDGES[case]
+    rng = np.random.default_rng(50 + case)
+    q = rng.standard_normal((H, T, D)).astype(np.float32)
+    k = core.f32_to_f16_bits(rng.standard_normal((Hkv, n_kv, D)).astype(np.float32))
+    v = core.f32_to_f16_bits(rng.standard_normal((Hkv, n_kv, D)).astype(np.float32))
+    m = np.where(rng.random((1, T, n_kv)) < 0.5, 0.0, -np.inf).astype(np.float32)
+    m[0, :, 0] = 0.5
+    mask = core.f32_to_f16_bits(m)
+    print("flash_attn edge %d: H=%d Hkv=%d T=%d D=%d n_kv=%d" % (case, H, Hkv, T, D, n_kv),
+          flush=True)
+    got = gpu_flash(L, q, k, v, Hkv, n_kv, (D, n_kv * D), (D, n_kv * D), mask, D ** -0.5)
+    want = core.flash_attn(q, k, v, Hkv, mask, D ** -0.5, 0.0, 0.0)
+    assert rel_err(got.reshape(T * H, D), want.reshape(T * H, D)) < 1e-5
+
+
+@pytest.mark.parametrize("T", [3, 500])
+def test_flash_attn_masked_cells_hold_anything(L, T):
+    """Cells that a row does not see may hold infinities and NaN in K and V;
+    a V value that is not finite reaches exactly the rows that see its cell;
+    rows whose every mask value is f16's lowest; f32 rows of q beyond f16."""
+    rng = np.random.default_rng(60)
+    H, Hkv, D, n_kv = 16, 8, 64, 150
+    q = rng.standard_normal((H, T, D)).astype(np.float32)
+    q[1] *= 3e5
+    k = rng.standard_normal((Hkv, n_kv, D)).astype(np.float32)
+    k[2:4] *= 1e-5  # heads 4..7: scores in range at q scaled up
+    v = rng.standard_normal((Hkv, n_kv, D)).astype(np.float32)
+    m = np.where(rng.random((1, T, n_kv)) < 0.3, -np.inf, 0.0).astype(np.float32)
+    m[0, :, 100:] = -np.inf
+    m[0, 0, :100] = -65504.0
+    m[0, :, 5] = 0.0
+    m[0, 1, 5] = -np.inf
+    clean = core.flash_attn(q, core.f32_to_f16_bits(k), core.f32_to_f16_bits(v), Hkv,
+                            core.f32_to_f16_bits(m), 0.125, 0.0, 0.0)
+    k[:, 100:], v[:, 100:] = np.nan, np.inf
+    v[:, 120] = np.nan
+    v[0, 5, 7] = np.inf  # heads 0 and 1, every row but row 1
+    got = gpu_flash(L, q, core.f32_to_f16_bits(k), core.f32_to_f16_bits(v), Hkv, n_kv,
+                    (D, n_kv * D), (D, n_kv * D), core.f32_to_f16_bits(m), 0.125)
+    sees = np.ones((T, H), bool)
+    sees[1] = False
+    sees[:, 2:] = False
+    # rows of head 1 put all weight on one cell: whether p of cell 5 is
+    # above 0 is theirs, so only head 0 is asserted to hold the infinity
+    assert np.isinf(got[sees[:, 0], 0, 7]).all() and np.isfinite(got[1]).all()
+    got[:, :2, 7], clean[:, :2, 7] = 0, 0
+    assert rel_err(got.reshape(T * H, D), clean.reshape(T * H, D)) < 1e-5
+
+
+def test_flash_attn_addresses_of_elements(L):
+    """q, v, the mask and out start at any element (k is 16-byte aligned)."""
+    from lgml_amd import hip
+    rng = np.random.default_rng(61)
+    H, Hkv, T, D, n_kv = 4, 2, 20, 48, 77
+    q = rng.standard_normal((H, T, D)).astype(np.float32)
+    k = core.f32_to_f16_bits(rng.standard_normal((Hkv, n_kv, D)).astype(np.float32))
+    v = core.f32_to_f16_bits(rng.standard_normal((Hkv, n_kv, D + 1)).astype(np.float32))
+    m = core.f32_to_f16_bits(np.where(rng.random((1, T, n_kv)) < 0.5, 0, -1).astype(np.float32))
+    qd, kd = dev(np.concatenate([np.zeros(1, np.float32), q.ravel()])), dev(k)
+    vd = dev(np.concatenate([np.zeros(1, np.uint16), v.ravel()]).view(np.int16))
+    md = dev(np.concatenate([np.zeros(3, np.uint16), m.ravel()]).view(np.int16))
+    out = torch.zeros(T * H * D + 1, dtype=torch.float32, device="cuda")
+    hip.check(L.lgmlh_flash_attn(qd.data_ptr() + 4, H, T, D, kd.data_ptr(), vd.data_ptr() + 2, Hkv,
+                                 n_kv, D, n_kv * D, D + 1, n_kv * (D + 1), md.data_ptr() + 6, 1, T,
+                                 0.2, 0.0, 0.0, out.data_ptr() + 4, st()))
+    want = core.flash_attn(q, k, np.ascontiguousarray(v[:, :, :D]), Hkv, m, 0.2, 0.0, 0.0)
+    got = out.cpu().numpy()
+    assert got[0] == 0
+    assert rel_err(got[1:].reshape(T * H, D), want.reshape(T * H, D)) < 1e-5
