@@ -16,6 +16,10 @@ typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 
+// f32 vectors that start at any element (the hardware loads such addresses,
+// and aligned ones as fast as ever).
+typedef f32x4 f32x4_u __attribute__((aligned(4)));
+
 namespace lgmlh {
 
 // Thread-local error text behind lgmlh_last_error().

@@ -55,7 +55,6 @@ __device__ __forceinline__ float alibi(int h, int H, float max_bias) {
 // out start anywhere their elements may; the hardware loads such addresses,
 // and aligned ones as fast as ever).
 typedef float f32x2 __attribute__((ext_vector_type(2)));
-typedef f32x4 f32x4_u __attribute__((aligned(4)));
 typedef u32x4 u32x4_u __attribute__((aligned(2)));
 typedef u32x2 u32x2_u __attribute__((aligned(2)));
 

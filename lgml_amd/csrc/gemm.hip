@@ -1263,28 +1263,88 @@ __global__ void xsplit_kernel(const void *__restrict__ x, int xtype, int64_t N, 
   act_store8(xf, planes, Npad, K, n, k0, v);
 }
 
-// ---- f32 weights: LDS-tiled VALU GEMM, sequential k order ----------------------
-__global__ void __launch_bounds__(256)
-f32gemm_kernel(const float *__restrict__ w, int64_t M, int64_t K, const float *__restrict__ x,
-               int64_t N, float *__restrict__ y, int64_t ldy, const float *__restrict__ residual) {
-  __shared__ float ws_[16][17], xs_[16][17];
-  const int tx = threadIdx.x & 15, ty = threadIdx.x >> 4;
-  const int64_t m = (int64_t)blockIdx.x * 16 + tx, n = (int64_t)blockIdx.y * 16 + ty;
-  float acc = 0.0f;
-  for (int64_t k0 = 0; k0 < K; k0 += 16) {
-    int64_t wm = (int64_t)blockIdx.x * 16 + ty, xn = (int64_t)blockIdx.y * 16 + ty;
-    ws_[ty][tx] = (wm < M && k0 + tx < K) ? w[wm * K + k0 + tx] : 0.0f;
-    xs_[ty][tx] = (xn < N && k0 + tx < K) ? x[xn * K + k0 + tx] : 0.0f;
-    __syncthreads();
+// ---- f32 weights: 16x16x4 f32 MFMAs ---------------------------------------------
+// K in chunks of 16 values (zeros past K): lane (row r16, quad) holds values
+// 4 quad .. 4 quad + 3 of a row's chunk, one 16-byte load, and MFMA j of a
+// chunk takes value j of every quad, so W and X feed the MFMAs as they lie
+// in memory. The chunks form at most F32_SEGS segments of equal length (from
+// K only); a segment's sum is one MFMA chain, the segments add in order,
+// then the residual: an element has the same bits at any N.
+//
+// A workgroup takes 16 x 16 outputs, a wave one segment of K. Products of few
+// outputs (routers, decode steps of small models) are a latency chain over
+// K, which the segments cut by 8: 128 x 2048 at 64 rows 52.6 us as one thread
+// per output with k in turn, 9.7 here (of which about 4.5 the launch); at
+// many outputs L2 bounds it, each tile reading its rows again: 2048 x 4096
+// at 576 rows 628 -> 255 us, 38 TFLOP/s (64 x 64 tiles of four waves reached
+// 39 there and 11 against 36 at 64 rows). The segments' sums are nearer to 64
+// bits than one chain over K: 9e-7 -> 3.2e-7 at K = 4096.
+constexpr int F32_SEGS = 8;
+
+__host__ __device__ inline int f32_seg_chunks(int64_t K) {
+  const int64_t c = (K + 15) / 16;
+  return (int)((c + F32_SEGS - 1) / F32_SEGS);
+}
+// Values k .. k + 3 of a row of K (zeros past K).
+__device__ __forceinline__ f32x4 f32_load4(const float *row, int64_t k, int64_t K) {
+  if (k + 4 <= K) return *(const f32x4_u *)(row + k);
+  f32x4 v = {0, 0, 0, 0};
 #pragma unroll
-    for (int k = 0; k < 16; k++) acc = fmaf(xs_[ty][k], ws_[tx][k], acc);
-    __syncthreads();
+  for (int i = 0; i < 4; i++)
+    if (k + i < K) v[i] = row[k + i];
+  return v;
+}
+// acc + the product of a chunk: D[m = 4 quad + i][n = r16].
+__device__ __forceinline__ f32x4 f32_chunk(f32x4 a, f32x4 b, f32x4 acc) {
+#pragma unroll
+  for (int j = 0; j < 4; j++) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a[j], b[j], acc, 0, 0, 0);
+  return acc;
+}
+__device__ __forceinline__ void f32_store4(f32x4 v, int64_t M, int64_t m, float *y,
+                                           const float *residual) {
+  if (m + 4 <= M) {
+    if (residual) v += *(const f32x4_u *)residual;
+    *(f32x4_u *)y = v;
+    return;
   }
-  if (m < M && n < N) {
-    float v = acc;
-    if (residual) v += residual[n * ldy + m];
-    y[n * ldy + m] = v;
+  for (int i = 0; i < 4; i++)
+    if (m + i < M) y[i] = residual ? v[i] + residual[i] : v[i];
+}
+
+__global__ void __launch_bounds__(64 * F32_SEGS)
+f32_split_kernel(const float *__restrict__ w, int64_t M, int64_t K, const float *__restrict__ x,
+                 int64_t N, float *y, int64_t ldy, const float *residual) {
+  __shared__ f32x4 part[F32_SEGS][64];
+  const int lane = threadIdx.x & 63, seg = threadIdx.x >> 6;
+  const int r16 = lane & 15, quad = lane >> 4;
+  const int64_t m0 = (int64_t)blockIdx.x * 16, n0 = (int64_t)blockIdx.y * 16;
+  const int64_t mr = m0 + r16 < M ? m0 + r16 : M - 1, nr = n0 + r16 < N ? n0 + r16 : N - 1;
+  const float *wr = w + mr * K, *xr = x + nr * K;
+  const int len = f32_seg_chunks(K);
+  const int64_t chunks = (K + 15) / 16, lo = (int64_t)seg * len;
+  const int64_t hi = lo + len < chunks ? lo + len : chunks;
+  f32x4 acc = {0, 0, 0, 0};
+  int64_t c = lo;
+  for (; c + 8 <= hi && (c + 8) * 16 <= K; c += 8) {  // eight chunks' loads in flight
+    f32x4 a[8], b[8];
+#pragma unroll
+    for (int u = 0; u < 8; u++) {
+      a[u] = *(const f32x4_u *)(wr + (c + u) * 16 + 4 * quad);
+      b[u] = *(const f32x4_u *)(xr + (c + u) * 16 + 4 * quad);
+    }
+#pragma unroll
+    for (int u = 0; u < 8; u++) acc = f32_chunk(a[u], b[u], acc);
   }
+  for (; c < hi; c++)
+    acc = f32_chunk(f32_load4(wr, c * 16 + 4 * quad, K), f32_load4(xr, c * 16 + 4 * quad, K), acc);
+  part[seg][lane] = acc;
+  __syncthreads();
+  if (seg != 0) return;
+  f32x4 v = acc;
+  const int nseg = (int)((chunks + len - 1) / len);
+  for (int s = 1; s < nseg; s++) v += part[s][lane];
+  const int64_t m = m0 + 4 * quad, n = n0 + r16;
+  if (n < N) f32_store4(v, M, m, y + n * ldy + m, residual ? residual + n * ldy + m : nullptr);
 }
 
 // K splits depend on M and K only, never on N: each output element is then
@@ -1542,7 +1602,8 @@ int mul_mat_f32(const float *w, int64_t M, int64_t K, const float *x, int64_t N,
   }
   if (N == 0) return LGMLH_OK;
   dim3 grid((unsigned)((M + 15) / 16), (unsigned)((N + 15) / 16));
-  hipLaunchKernelGGL(f32gemm_kernel, grid, dim3(256), 0, st, w, M, K, x, N, y, ldy, residual);
+  hipLaunchKernelGGL(f32_split_kernel, grid, dim3(64 * F32_SEGS), 0, st, w, M, K, x, N, y, ldy,
+                     residual);
   return hip_check(hipGetLastError(), "mul_mat");
 }
 

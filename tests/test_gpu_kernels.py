@@ -380,3 +380,28 @@ def test_plan_cells_and_errors(L):
         runtime.Plan([3, 2], [126, 127], bt, np.zeros(5, np.int32), 4, 2, 16)  # seq 1 needs a 3rd block
     with pytest.raises(hip.LgmlhError):
         runtime.Plan([3], [126], bt[:1], np.zeros(3, np.int32), 4, 2, 9)  # block 9 past the pool
+
+
+# f32 products at the edges of the 16 x 16 tiles, the chunks of 16 and the
+# eight segments of K. A sum of K f32 products is within (K / 8 + 16) 2^-24 of
+# the sum of their magnitudes (a segment's chain, then the segments), which
+# for random signs is at most sqrt(K) times the result's rms here.
+@pytest.mark.parametrize("M,K,N", [(1, 1, 1), (16, 16, 16), (17, 15, 3), (33, 130, 65),
+                                   (5, 2049, 40), (128, 2048, 64), (64, 4099, 17)])
+def test_f32_product_edges_and_batch_invariance(L, M, K, N):
+    from lgml_amd import hip
+    rng = np.random.default_rng(M + K)
+    w, x = rng.standard_normal((M, K)).astype(np.float32), rng.standard_normal((N, K)).astype(np.float32)
+    r = rng.standard_normal((N, M)).astype(np.float32)
+    wd, xd, rd = dev(w), dev(x), dev(r)
+    y, one = torch.empty((N, M), device="cuda"), torch.empty((1, M), device="cuda")
+    hip.check(L.lgmlh_mul_mat(core.F32, wd.data_ptr(), M, K, xd.data_ptr(), hip.F32, N, y.data_ptr(),
+                              hip.EPI_ADD, rd.data_ptr(), None, 0, st()))
+    want = x.astype(np.float64) @ w.astype(np.float64).T + r
+    bound = (K / 8 + 16) * 2.0 ** -24 * np.sqrt(K) * 4
+    assert np.abs(y.cpu().numpy() - want).max() <= max(bound, 1e-6) * np.sqrt(np.mean(want ** 2))
+    for j in (0, N - 1):  # a row alone gives the same bits
+        hip.check(L.lgmlh_mul_mat(core.F32, wd.data_ptr(), M, K, xd[j:j + 1].data_ptr(), hip.F32, 1,
+                                  one.data_ptr(), hip.EPI_ADD, rd[j:j + 1].data_ptr(), None, 0,
+                                  st()))
+        assert torch.equal(one[0], y[j])
