@@ -22,6 +22,20 @@ typedef f32x4 f32x4_u __attribute__((aligned(4)));
 
 namespace lgmlh {
 
+// The launch of an elementwise kernel over n rows of `per_row` threads each:
+// threads along the row in whole waves (blocks of up to 256, several short
+// rows to a block), rows in blockIdx.y and threadIdx.y; a grid of at most
+// 65535 in y, past which the kernel's row loop goes on.
+struct RowGrid {
+  dim3 grid, block;
+  RowGrid(int64_t per_row, int64_t n) {
+    const int64_t bx = per_row > 128 ? 256 : per_row > 64 ? 128 : 64;
+    const int64_t by = 256 / bx, gy = (n + by - 1) / by;
+    block = dim3((unsigned)bx, (unsigned)by);
+    grid = dim3((unsigned)((per_row + bx - 1) / bx), (unsigned)(gy < 65535 ? gy : 65535));
+  }
+};
+
 // Thread-local error text behind lgmlh_last_error().
 void set_error(const char *fmt, ...);
 

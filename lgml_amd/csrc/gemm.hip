@@ -1228,13 +1228,25 @@ qstream_kernel(const uint8_t *__restrict__ w, int64_t M, int64_t K, const f16 *_
 // residual.
 __global__ void splitk_reduce_kernel(Pending pd, float *__restrict__ y, int64_t ldy,
                                      const float *__restrict__ residual) {
-  const int64_t total = pd.rows * pd.cols, M = pd.cols;
-  for (int64_t e = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; e < total;
-       e += (int64_t)gridDim.x * blockDim.x) {
-    int64_t n = e / M, m = e % M;
-    float v = pd.sum(n, m);
-    if (residual) v += residual[n * ldy + m];
-    y[n * ldy + m] = v;
+  const int64_t M = pd.cols, m = 4 * (blockIdx.x * (int64_t)blockDim.x + threadIdx.x);
+  if (m >= M) return;
+  const bool vec = (M & 3) == 0;  // 4 columns a thread; rows of partials then start at 16 bytes
+  for (int64_t n = blockIdx.y * (int64_t)blockDim.y + threadIdx.y; n < pd.rows;
+       n += (int64_t)gridDim.y * blockDim.y) {
+    float *yr = y + n * ldy + m;
+    const float *rr = residual ? residual + n * ldy + m : nullptr;
+    if (vec) {
+      float v[4];
+      pd.sum4(n, m, v);
+      f32x4 o = {v[0], v[1], v[2], v[3]};
+      if (rr) o += *(const f32x4_u *)rr;
+      *(f32x4_u *)yr = o;
+    } else {
+      for (int e = 0; e < 4 && m + e < M; e++) {
+        const float v = pd.sum(n, m + e);
+        yr[e] = rr ? v + rr[e] : v;
+      }
+    }
   }
 }
 
@@ -1242,25 +1254,26 @@ __global__ void splitk_reduce_kernel(Pending pd, float *__restrict__ y, int64_t 
 // (the lanes of a 256-value block are consecutive and leave together).
 __global__ void xsplit_kernel(const void *__restrict__ x, int xtype, int64_t N, int64_t K,
                               f16 *__restrict__ planes, int64_t Npad, int xf) {
-  const int64_t per_row = K / 8;  // a multiple of 32: groups never straddle rows
-  const int64_t t = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-  if (t >= N * per_row) return;   // whole groups of 4 lanes leave together
-  const int64_t n = t / per_row, k0 = (t % per_row) * 8;
-  float v[8];
-  if (xtype == LGMLH_F32) {
-    const f32x4 *p = (const f32x4 *)((const float *)x + n * K + k0);
-    f32x4 a = p[0], b = p[1];
+  const int64_t k0 = 8 * (blockIdx.x * (int64_t)blockDim.x + threadIdx.x);
+  if (k0 >= K) return;  // K % 256 == 0: whole blocks of lanes leave together
+  for (int64_t n = blockIdx.y * (int64_t)blockDim.y + threadIdx.y; n < N;
+       n += (int64_t)gridDim.y * blockDim.y) {
+    float v[8];
+    if (xtype == LGMLH_F32) {
+      const f32x4 *p = (const f32x4 *)((const float *)x + n * K + k0);
+      f32x4 a = p[0], b = p[1];
 #pragma unroll
-    for (int e = 0; e < 4; e++) {
-      v[e] = a[e];
-      v[4 + e] = b[e];
+      for (int e = 0; e < 4; e++) {
+        v[e] = a[e];
+        v[4 + e] = b[e];
+      }
+    } else {
+      f16x8 h = *(const f16x8 *)((const f16 *)x + n * K + k0);
+#pragma unroll
+      for (int e = 0; e < 8; e++) v[e] = (float)h[e];
     }
-  } else {
-    f16x8 h = *(const f16x8 *)((const f16 *)x + n * K + k0);
-#pragma unroll
-    for (int e = 0; e < 8; e++) v[e] = (float)h[e];
+    act_store8(xf, planes, Npad, K, n, k0, v);
   }
-  act_store8(xf, planes, Npad, K, n, k0, v);
 }
 
 // ---- f32 weights: 16x16x4 f32 MFMAs ---------------------------------------------
@@ -1411,11 +1424,10 @@ static int launch_q(const void *w, int64_t M, int64_t K, const f16 *xs, int64_t 
 #undef LGMLH_STREAM
       *group = SPLIT_PAIR;
       if (splits > 1 && !defer) {
-        int64_t total = N * M;
-        unsigned blocks = (unsigned)((total + 255) / 256 < 4096 ? (total + 255) / 256 : 4096);
         Pending pd{part, splits, N, M};
         pd.group = SPLIT_PAIR;
-        hipLaunchKernelGGL(splitk_reduce_kernel, dim3(blocks), dim3(256), 0, st, pd, y, ldy, res);
+        const RowGrid g((M + 3) / 4, N);
+        hipLaunchKernelGGL(splitk_reduce_kernel, g.grid, g.block, 0, st, pd, y, ldy, res);
       }
       return splits > 1 ? splits : 0;
     }
@@ -1462,11 +1474,10 @@ static int launch_q(const void *w, int64_t M, int64_t K, const f16 *xs, int64_t 
     LGMLH_PLAIN(4);
 #undef LGMLH_PLAIN
   if (nz > 1 && !defer) {
-    int64_t total = N * M;
-    unsigned blocks = (unsigned)((total + 255) / 256 < 4096 ? (total + 255) / 256 : 4096);
     Pending pd{part, nz, N, M};
     pd.group = *group;
-    hipLaunchKernelGGL(splitk_reduce_kernel, dim3(blocks), dim3(256), 0, st, pd, y, ldy, res);
+    const RowGrid g((M + 3) / 4, N);
+    hipLaunchKernelGGL(splitk_reduce_kernel, g.grid, g.block, 0, st, pd, y, ldy, res);
   }
   return nz > 1 ? nz : 0;
 }
@@ -1586,10 +1597,9 @@ int split_x(const void *x, int xtype, int64_t N, int64_t K, f16 *xs, hipStream_t
     set_error("split: bad arguments");
     return LGMLH_EINVAL;
   }
-  int64_t total = N * (K / 8);
-  if (total == 0) return LGMLH_OK;
-  hipLaunchKernelGGL(xsplit_kernel, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, st, x,
-                     xtype, N, K, xs, split_npad(N), xf);
+  if (N * K == 0) return LGMLH_OK;
+  const RowGrid g(K / 8, N);
+  hipLaunchKernelGGL(xsplit_kernel, g.grid, g.block, 0, st, x, xtype, N, K, xs, split_npad(N), xf);
   return hip_check(hipGetLastError(), "split");
 }
 

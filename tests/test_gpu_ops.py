@@ -293,3 +293,45 @@ def test_gen_normal_matches_oracle(L, case):
     else:
         want = core.gen_normal_quant(ty, rows, cols, mean, sd, seed).reshape(-1)
     assert np.array_equal(got, want)
+
+
+# rows that are not whole vectors of 4, several rows to a workgroup, more
+# columns than one; f32 and f16 outputs. The unit is f64 rounded once (one
+# f32 ulp covers the f64 function's own error).
+@pytest.mark.parametrize("n,F", [(1, 1), (3, 5), (7, 258), (5, 1027), (2, 4096)])
+@pytest.mark.parametrize("gelu", [0, 1])
+def test_gated_unit_row_edges(L, n, F, gelu):
+    from lgml_amd import hip
+    rng = np.random.default_rng(F)
+    gu = (rng.standard_normal((n, 2 * F)) * 4).astype(np.float32)
+    gu[0, 0] = -700.0
+    g, u = gu[:, :F].astype(np.float64), gu[:, F:].astype(np.float64)
+    z = 2 * np.sqrt(2 / np.pi) * (g + 0.044715 * g ** 3) if gelu else g
+    with np.errstate(over="ignore"):
+        want = g / (1 + np.exp(-z)) * u
+    d = dev(gu)
+    fn = L.lgmlh_geglu if gelu else L.lgmlh_swiglu
+    out = torch.empty((n, F), device="cuda")
+    hip.check(fn(d.data_ptr(), n, F, out.data_ptr(), hip.F32, st()))
+    got = out.cpu().numpy()
+    assert (np.abs(got - want) <= 2.0 ** -23 * np.abs(want) + 1e-38).all()
+    half = torch.empty((n, F), dtype=torch.float16, device="cuda")
+    hip.check(fn(d.data_ptr(), n, F, half.data_ptr(), hip.F16, st()))
+    assert np.array_equal(half.cpu().numpy().view(np.uint16), got.astype(np.float16).view(np.uint16))
+
+
+@pytest.mark.parametrize("n", [1, 3, 4, 4095, 32768, 32773, 131072 + 2])
+def test_argmax_row_edges(L, n):
+    from lgml_amd import hip
+    rng = np.random.default_rng(n)
+    x = rng.standard_normal((4, n)).astype(np.float32)
+    x[0, n - 1] = 9.0
+    x[1, n // 2:] = 9.0  # ties: the first
+    x[2] = -np.inf       # nothing above -inf: index 0
+    x[3, 0] = -np.inf
+    if n > 2:
+        x[3, 1:] = np.nan
+        x[3, 2] = -5.0
+    d, out = dev(x), torch.empty(4, dtype=torch.int32, device="cuda")
+    hip.check(L.lgmlh_argmax(d.data_ptr(), 4, n, out.data_ptr(), st()))
+    assert out.cpu().tolist() == [n - 1, n // 2, 0, 2 if n > 2 else 0]
