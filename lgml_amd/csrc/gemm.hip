@@ -22,6 +22,7 @@
 // workgroups when M alone gives too few (split count from M and K only);
 // the splits are added in a fixed order by a second kernel.
 #include <mutex>
+#include <type_traits>
 
 #include "common.h"
 #include "quant.h"
@@ -463,10 +464,11 @@ qgemm_kernel(const uint8_t *__restrict__ w, int64_t M, int64_t K, const f16 *__r
   }
   // Q8_0 header piece of lane < 32: tile lane / 16, bytes 16 (lane % 16)
   const uint8_t *hsrc = wt[(lane >> 4) & 1] + 16 * (lane & 15);
-  auto load_x = [&](uint32_t kstep, int buf) {  // kstep = sb - sb_lo
+  auto load_x = [&](uint32_t kstep, int buf, int live) {  // kstep = sb - sb_lo
 #pragma unroll
     for (int j = 0; j < XJ; j++) {
       const int slot0 = (wave * XJ + j) * 64;
+      if (NCT == 4 && GATHER && slot0 >= live * 16 * 32) continue;  // a column tile without picks
       // a wave-uniform base plus a 32-bit lane offset (no 64-bit adds per lane)
       const uint8_t *bh = (const uint8_t *)(xhi + kstep * QK_K);
       const uint8_t *bl = (const uint8_t *)(xlo + kstep * QK_K);
@@ -510,17 +512,21 @@ qgemm_kernel(const uint8_t *__restrict__ w, int64_t M, int64_t K, const f16 *__r
   };
   const uint32_t sh6 = 8u * (uint32_t)(c >> 1);
 
+  // The column tiles in use (GATHER: a 64-column tile often holds fewer picks;
+  // the tiles past them are neither loaded nor multiplied).
+  auto run = [&](auto live_) __attribute__((always_inline)) {
+  constexpr int LIVE = decltype(live_)::value;
   // One K step on the staged X with the weight fragments cur. The B
   // fragments of group g + 1 are read while group g multiplies; within a
   // group the products with hi go before those with lo, so no MFMA waits
   // for the one just issued.
   auto compute = [&](const WFrag<TYPE>(&cur)[RT_PER_WAVE], int buf) {
     const u32x4 *xh = XH(buf), *xl = XL(buf);
-    f32x4 cm[RT_PER_WAVE][NCT];
+    f32x4 cm[RT_PER_WAVE][LIVE];
     // The two buffers are separate LDS objects, so the compiler lets these
     // reads run while the next step's global-to-LDS loads into the other
     // buffer are in flight.
-    f16x4 sh4[NCT], sl4[NCT];
+    f16x4 sh4[LIVE], sl4[LIVE];
     if constexpr (TYPE == LGMLH_Q4_K && !Q8) {
       // lanes c >= 2 (k past the 8 groups) read zeros: no branch per step
       const bool gs = c < 2;
@@ -528,7 +534,7 @@ qgemm_kernel(const uint8_t *__restrict__ w, int64_t M, int64_t K, const f16 *__r
       const f16 *gl = gh + (gs ? 64 * 8 : 0);
       const int cstride = gs ? 16 * 8 : 0;
 #pragma unroll
-      for (int ct = 0; ct < NCT; ct++) {
+      for (int ct = 0; ct < LIVE; ct++) {
         sh4[ct] = *(const f16x4 *)(gh + ct * cstride);
         sl4[ct] = *(const f16x4 *)(gl + ct * cstride);
       }
@@ -537,7 +543,7 @@ qgemm_kernel(const uint8_t *__restrict__ w, int64_t M, int64_t K, const f16 *__r
       // the 16 sums of 16 q: lane c holds sums 4c .. 4c + 3 of its column
       const f16 *gs = (const f16 *)GS(buf) + (c < 2 ? 0 : 64 * 8) + r16 * 8 + 4 * (c & 1);
 #pragma unroll
-      for (int ct = 0; ct < NCT; ct++) sh4[ct] = *(const f16x4 *)(gs + ct * 16 * 8);
+      for (int ct = 0; ct < LIVE; ct++) sh4[ct] = *(const f16x4 *)(gs + ct * 16 * 8);
     }
     uint32_t scb[RT_PER_WAVE][2];
     if constexpr (TYPE == LGMLH_Q4_K) {
@@ -549,17 +555,17 @@ qgemm_kernel(const uint8_t *__restrict__ w, int64_t M, int64_t K, const f16 *__r
     }
     // B fragments: a group's hi (lo) fragments are read right after the
     // previous group's products with hi (lo) are issued.
-    f16x8 bh[NCT], bl[NCT];
+    f16x8 bh[LIVE], bl[LIVE];
     auto read_bh = [&](int g) {
       const int slot = r16 * 32 + ((4 * g + c) ^ r16);
 #pragma unroll
-      for (int ct = 0; ct < NCT; ct++) bh[ct] = __builtin_bit_cast(f16x8, xh[ct * 16 * 32 + slot]);
+      for (int ct = 0; ct < LIVE; ct++) bh[ct] = __builtin_bit_cast(f16x8, xh[ct * 16 * 32 + slot]);
     };
     auto read_bl = [&](int g) {
       if constexpr (!Q8) {
         const int slot = r16 * 32 + ((4 * g + c) ^ r16);
 #pragma unroll
-        for (int ct = 0; ct < NCT; ct++) bl[ct] = __builtin_bit_cast(f16x8, xl[ct * 16 * 32 + slot]);
+        for (int ct = 0; ct < LIVE; ct++) bl[ct] = __builtin_bit_cast(f16x8, xl[ct * 16 * 32 + slot]);
       }
     };
     // Q8_0: d of rows 4c .. 4c + 3 of tile a, block g
@@ -598,7 +604,7 @@ qgemm_kernel(const uint8_t *__restrict__ w, int64_t M, int64_t K, const f16 *__r
 #pragma unroll
       for (int a = 0; a < RT_PER_WAVE; a++)
 #pragma unroll
-        for (int ct = 0; ct < NCT; ct++) {
+        for (int ct = 0; ct < LIVE; ct++) {
           const f32x4 c0 = (g == 0 || TYPE == LGMLH_Q8_0) ? f32x4{0, 0, 0, 0} : cm[a][ct];
           cm[a][ct] = __builtin_amdgcn_mfma_f32_16x16x32_f16(af[a], bh[ct], c0, 0, 0, 0);
         }
@@ -606,7 +612,7 @@ qgemm_kernel(const uint8_t *__restrict__ w, int64_t M, int64_t K, const f16 *__r
 #pragma unroll
         for (int a = 0; a < RT_PER_WAVE; a++)
 #pragma unroll
-          for (int ct = 0; ct < NCT; ct++)
+          for (int ct = 0; ct < LIVE; ct++)
             cm[a][ct] = __builtin_amdgcn_mfma_f32_16x16x32_f16(af2[a], bh[ct], cm[a][ct], 0, 0, 0);
       }
       if (g < 7) read_bh(g + 1);
@@ -614,7 +620,7 @@ qgemm_kernel(const uint8_t *__restrict__ w, int64_t M, int64_t K, const f16 *__r
 #pragma unroll
         for (int a = 0; a < RT_PER_WAVE; a++)
 #pragma unroll
-          for (int ct = 0; ct < NCT; ct++)
+          for (int ct = 0; ct < LIVE; ct++)
             cm[a][ct] = __builtin_amdgcn_mfma_f32_16x16x32_f16(
                 TYPE == LGMLH_Q6_K ? afr[a] : af[a], bl[ct], cm[a][ct], 0, 0, 0);
         if (g < 7) read_bl(g + 1);
@@ -626,10 +632,10 @@ qgemm_kernel(const uint8_t *__restrict__ w, int64_t M, int64_t K, const f16 *__r
       if constexpr (TYPE == LGMLH_Q8_0) {
         // one scale per 32-value block: flush every group (Q8: times the
         // column's d of the block, (d_w d_x) I as ggml's q8_0 dot)
-        float dxg[NCT];
+        float dxg[LIVE];
         if constexpr (Q8) {
 #pragma unroll
-          for (int ct = 0; ct < NCT; ct++)
+          for (int ct = 0; ct < LIVE; ct++)
             dxg[ct] = DX(buf)[(g >> 2) * 256 + (ct * 16 + r16) * 4 + (g & 3)];
         }
 #pragma unroll
@@ -638,7 +644,7 @@ qgemm_kernel(const uint8_t *__restrict__ w, int64_t M, int64_t K, const f16 *__r
           for (int i = 0; i < 4; i++) {
             const float d = h2f((uint16_t)(dg[a][i >> 1] >> (16 * (i & 1))));
 #pragma unroll
-            for (int ct = 0; ct < NCT; ct++) {
+            for (int ct = 0; ct < LIVE; ct++) {
               if constexpr (Q8)
                 acc[a][ct][i] = fmaf(d * dxg[ct], cm[a][ct][i], acc[a][ct][i]);
               else
@@ -652,14 +658,14 @@ qgemm_kernel(const uint8_t *__restrict__ w, int64_t M, int64_t K, const f16 *__r
 #pragma unroll
         for (int a = 0; a < RT_PER_WAVE; a++)
 #pragma unroll
-          for (int ct = 0; ct < NCT; ct++) asm volatile("" : "+v"(acc[a][ct]));
+          for (int ct = 0; ct < LIVE; ct++) asm volatile("" : "+v"(acc[a][ct]));
       }
     }
     // Q8 (Q8_K): the column's d of this K step
-    float dxs[NCT];
+    float dxs[LIVE];
     if constexpr (Q8 && TYPE != LGMLH_Q8_0) {
 #pragma unroll
-      for (int ct = 0; ct < NCT; ct++) dxs[ct] = DX(buf)[ct * 16 + r16];
+      for (int ct = 0; ct < LIVE; ct++) dxs[ct] = DX(buf)[ct * 16 + r16];
     }
     if constexpr (TYPE == LGMLH_Q4_K) {
       // min term: sum_g m_g * S_g[n] as a 16x16x16 MFMA over the 8 groups
@@ -674,7 +680,7 @@ qgemm_kernel(const uint8_t *__restrict__ w, int64_t M, int64_t K, const f16 *__r
           dm[i] = h2f((uint16_t)(cur[a].dm[i] >> 16));
         }
 #pragma unroll
-        for (int ct = 0; ct < NCT; ct++) {
+        for (int ct = 0; ct < LIVE; ct++) {
           f32x4 mn = __builtin_amdgcn_mfma_f32_16x16x16f16(am, sh4[ct], f32x4{0, 0, 0, 0}, 0, 0, 0);
           if constexpr (!Q8) {
             mn = __builtin_amdgcn_mfma_f32_16x16x16f16(am, sl4[ct], mn, 0, 0, 0);
@@ -698,7 +704,7 @@ qgemm_kernel(const uint8_t *__restrict__ w, int64_t M, int64_t K, const f16 *__r
           // the fragments carry sc * q / 4
           const float d4 = 4.0f * h2f((uint16_t)(cur[a].d4[i >> 1] >> (16 * (i & 1))));
 #pragma unroll
-          for (int ct = 0; ct < NCT; ct++) {
+          for (int ct = 0; ct < LIVE; ct++) {
             if constexpr (Q8)
               acc[a][ct][i] = fmaf(d4 * dxs[ct], cm[a][ct][i], acc[a][ct][i]);
             else
@@ -725,11 +731,11 @@ qgemm_kernel(const uint8_t *__restrict__ w, int64_t M, int64_t K, const f16 *__r
       // one buffer: the next step's X goes in once every wave has read it
       compute(cur, 0);
       __syncthreads();
-      load_x(kn, 0);
+      load_x(kn, 0, LIVE);
       __builtin_amdgcn_s_waitcnt(0);
       __syncthreads();
     } else {
-      load_x(kn, buf ^ 1);
+      load_x(kn, buf ^ 1, LIVE);
       compute(cur, buf);
       __builtin_amdgcn_s_waitcnt(0);  // this wave's X loads have landed in LDS
       __syncthreads();                // ... and everyone's; buffer buf is free again
@@ -737,7 +743,7 @@ qgemm_kernel(const uint8_t *__restrict__ w, int64_t M, int64_t K, const f16 *__r
   };
   if (nsteps > 0) {
     load_w(w0, 0);
-    load_x(0, 0);
+    load_x(0, 0, LIVE);
     __builtin_amdgcn_s_waitcnt(0);
     __syncthreads();
   }
@@ -762,7 +768,7 @@ qgemm_kernel(const uint8_t *__restrict__ w, int64_t M, int64_t K, const f16 *__r
 #pragma unroll
     for (int a = 0; a < RT_PER_WAVE; a++)
 #pragma unroll
-      for (int ct = 0; ct < NCT; ct++) {
+      for (int ct = 0; ct < LIVE; ct++) {
         int64_t n = n0 + ct * 16 + r16;
         int64_t m = (rt0 + a) * 16 + 4 * c;
         if constexpr (GATHER) {
@@ -799,7 +805,7 @@ qgemm_kernel(const uint8_t *__restrict__ w, int64_t M, int64_t K, const f16 *__r
 #pragma unroll
       for (int a = 0; a < RT_PER_WAVE; a++)
 #pragma unroll
-        for (int ct = 0; ct < NCT; ct++) acc[a][ct] = f32x4{0, 0, 0, 0};
+        for (int ct = 0; ct < LIVE; ct++) acc[a][ct] = f32x4{0, 0, 0, 0};
     }
   };
   for (uint32_t k = 0; k < nsteps; k += 2) {
@@ -814,6 +820,19 @@ qgemm_kernel(const uint8_t *__restrict__ w, int64_t M, int64_t K, const f16 *__r
     emit(out, ld_out, true, nz == 1 && residual);
   else
     emit(out, ld_out, false, nz == 1 && residual);
+  };
+  if constexpr (GATHER && NCT == 4) {
+    if (count > 48)
+      run(std::integral_constant<int, 4>{});
+    else if (count > 32)
+      run(std::integral_constant<int, 3>{});
+    else if (count > 16)
+      run(std::integral_constant<int, 2>{});
+    else
+      run(std::integral_constant<int, 1>{});
+  } else {
+    run(std::integral_constant<int, NCT>{});
+  }
 }
 
 // ---- decode-sized products: the weights stream through LDS ----------------------

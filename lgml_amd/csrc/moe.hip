@@ -664,10 +664,18 @@ __global__ void moe_sum_kernel(const float *__restrict__ y, const float *__restr
 static size_t a256(size_t b) { return (b + 255) & ~size_t(255); }
 
 // Column tile width for P picks over NE experts: 64 once an expert averages
-// 128 picks, else 16. (A 512-token prefill pass of C5 gives an expert about
-// 36 picks: in 64-column tiles those are half empty, and 16-column ones,
-// two workgroups per CU, made C5's mixed phase 9% faster.)
-int moe_tile_cols(int64_t P, int NE) { return P >= 128 * (int64_t)NE ? 64 : 16; }
+// 24 picks and there are 1024 of them (or it averages 128), else 16. A
+// 64-column tile works on its 16-column parts in use, so it builds an
+// expert's weight fragments once where 16-column tiles build them per 16
+// picks; 16-column ones run twice the waves per CU. (The MoE layer of 512 x 8
+// picks over 128 experts of 768 x 2048, 32 picks each: Q4_K 262 us in 16-
+// column tiles, 222 in 64-column ones, Q8_0 387 and 286; 16 picks each: 169
+// and 175; 8 experts with 32 picks each, too few tiles to fill the chip: 58
+// and 67.)
+int moe_tile_cols(int64_t P, int NE) {
+  const int64_t ne = NE;
+  return P >= 128 * ne || (P >= 24 * ne && P >= 1024) ? 64 : 16;
+}
 
 // An upper bound of the tiles of a grouping: sum over experts of
 // ceil(c_e / tc) <= (P + (tc - 1) * min(NE, P)) / tc, and <= P.

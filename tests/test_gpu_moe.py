@@ -172,3 +172,40 @@ def test_c5_batched_pass_equals_lone_pass():
     for s, p in enumerate(prompts):
         la = gm.forward(gm.plan([len(p)], [0], bt[s:s + 1], np.array(p, np.int32)))
         assert np.array_equal(la.cpu().numpy()[0].view(np.uint32), lb[s].view(np.uint32))
+
+
+@pytest.mark.parametrize("ty", [core.Q4_K, core.Q6_K, core.Q8_0])
+@pytest.mark.parametrize("ggml", [False, True])
+def test_grouped_product_tile_parts(ty, ggml):
+    """64-column tiles with every number of 16-column parts in use: experts
+    with 0, 1, 15 .. 17, 31 .. 33, 47 .. 49, 63 .. 65 and more picks (1024
+    picks in all, so that the wide tiles run)."""
+    from lgml_amd import hip
+    L = hip.lib()
+    counts = [0, 1, 15, 16, 17, 31, 32, 33, 47, 48, 49, 63, 64, 65, 128, 129, 200]
+    NE, M, K, nu = len(counts) + 2, 80, 512, 1
+    T = 2100
+    ids = np.concatenate([np.full(n, e) for e, n in enumerate(counts)])
+    ids = np.concatenate([ids, np.full((T - len(ids)) // 2, NE - 2)])
+    ids = np.concatenate([ids, np.full(T - len(ids), NE - 1)]).astype(np.int32)
+    rng = np.random.default_rng(5)
+    rng.shuffle(ids)
+    ids = ids.reshape(T, nu)
+    w = core.quantize(ty, core.fill_normal(NE * M * K, 0, 0.02, 31).reshape(NE * M, K))
+    x = core.fill_normal(T * K, 0, 1, 32).reshape(T, 1, K)
+    eb = L.lgmlh_repacked_bytes(ty, M, K)
+    rp = torch.empty(NE * eb, dtype=torch.uint8, device="cuda")
+    stream = torch.cuda.current_stream().cuda_stream
+    for e in range(NE):
+        src = torch.from_numpy(w[e * M:(e + 1) * M].copy()).cuda()
+        hip.check(L.lgmlh_repack(ty, M, K, src.data_ptr(), rp.data_ptr() + e * eb, stream))
+        torch.cuda.synchronize()
+    n = L.lgmlh_mul_mat_id_workspace(ty, NE, M, K, T, 1, nu)
+    ws = torch.empty(n, dtype=torch.uint8, device="cuda")
+    y = torch.empty((T, nu, M), device="cuda")
+    xd, idd = torch.from_numpy(x).cuda(), torch.from_numpy(ids).cuda()
+    fn = L.lgmlh_mul_mat_id_ggml if ggml else L.lgmlh_mul_mat_id
+    hip.check(fn(ty, rp.data_ptr(), NE, M, K, xd.data_ptr(), hip.F32, 1, idd.data_ptr(), T, nu,
+                 y.data_ptr(), ws.data_ptr(), n, stream))
+    want = core.mul_mat_id(ty, w, NE, M, K, x, ids, act_quant=ggml)
+    assert rel_err(y.cpu().numpy().reshape(T, M), want.reshape(T, M)) < 1e-5
