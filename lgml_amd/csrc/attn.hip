@@ -10,7 +10,7 @@
 // (K rows straight from the [cell][D] tile), an online softmax per row in
 // f32 (each lane owns one row; reductions over 4 lanes with shuffles), and
 // O^T += V^T P^T (V columns straight from the transposed [D][cell] tile, P
-// through 4.6 KB of LDS). K and V are exact f16; Q and P enter the MFMAs as
+// from the lane's own S^T values: s_cell). K and V are exact f16; Q and P enter the MFMAs as
 // f16 hi + lo pairs, so every product is f32-accurate. The loads of block
 // b + 1 are issued as soon as block b's registers are consumed (K after
 // S, V after O), so they overlap block b's softmax and products.
@@ -34,7 +34,6 @@
 namespace lgmlh {
 
 constexpr int ROWS = 16;      // MFMA rows per wave
-constexpr int P_STRIDE = 72;  // f16 per LDS row of P (64 cells + pad)
 constexpr float LOG2E = 1.4426950408889634f;
 
 __device__ __forceinline__ f32x4 mfma16(f16x8 a, f16x8 b, f32x4 c) {
@@ -43,6 +42,83 @@ __device__ __forceinline__ f32x4 mfma16(f16x8 a, f16x8 b, f32x4 c) {
 
 __device__ __forceinline__ f16x8 load_f16x8(const uint16_t *p) {
   return __builtin_bit_cast(f16x8, *(const u32x4 *)p);
+}
+
+// The cells of the S^T tiles. MFMA row r of tile ct is cell 32 (ct / 2) + 8 (r /
+// 4) + 4 (ct % 2) + r % 4 of the block: the 4 values that lane quad q holds of
+// tiles 2j and 2j + 1 are then cells 32 j + 8 q .. + 7, the B operand of the
+// second product over the V^T tile's own order of cells, and P never leaves
+// the registers. (With P through LDS and K and V fragments read as they were
+// needed, a 512-token chunk after 1024 tokens, 32 / 8 heads of 128, took 65.7
+// us; 59.6 here. 300 tokens beside 16 sequences, 8 / 4 heads of 64: 42.0 and
+// 34.6.)
+__device__ __forceinline__ int s_cell(int ct, int r) {
+  return 32 * (ct >> 1) + 8 * (r >> 2) + 4 * (ct & 1) + (r & 3);
+}
+
+// Scores of one block (scaled, in units of log2) -> P, the running max and
+// sum, and the rescale of O^T: the online softmax of a row (a lane owns one;
+// its quads hold the cells). masked: cells past p_row (RING: before the window)
+// are dropped; rows past the group hold zeros and are never stored.
+typedef float f32x2 __attribute__((ext_vector_type(2)));
+template <int DT>
+__device__ __forceinline__ void softmax_block(f32x4 (&st)[4], float scale_log2, bool full,
+                                              int cbase, int quad, int p_row, int p_lo, bool rvalid,
+                                              float &m, float &l, f32x4 (&o)[DT], f16x8 (&ph)[2],
+                                              f16x8 (&pl)[2]) {
+#pragma unroll
+  for (int ct = 0; ct < 4; ct++) st[ct] *= scale_log2;
+  if (!full) {  // wave-uniform
+#pragma unroll
+    for (int ct = 0; ct < 4; ct++)
+#pragma unroll
+      for (int i = 0; i < 4; i++) {
+        const int p = cbase + s_cell(ct, 4 * quad + i);
+        if (!rvalid || p > p_row || p < p_lo) st[ct][i] = -INFINITY;
+      }
+  }
+  float mx = -INFINITY;
+#pragma unroll
+  for (int ct = 0; ct < 4; ct++)
+#pragma unroll
+    for (int i = 0; i < 4; i++) mx = fmaxf(mx, st[ct][i]);
+  mx = fmaxf(mx, __shfl_xor(mx, 16));
+  mx = fmaxf(mx, __shfl_xor(mx, 32));
+  const float m_new = fmaxf(m, mx);
+  const float m_use = m_new == -INFINITY ? 0.0f : m_new;
+  float rs = 0.0f;
+#pragma unroll
+  for (int ct = 0; ct < 4; ct++)
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+      st[ct][i] = __builtin_amdgcn_exp2f(st[ct][i] - m_use);  // exp2(-inf) = 0
+      rs += st[ct][i];
+    }
+  rs += __shfl_xor(rs, 16);
+  rs += __shfl_xor(rs, 32);
+  // rescale only when some row's maximum moved
+  if (__builtin_amdgcn_ballot_w64(m_new != m)) {
+    const float alpha = __builtin_amdgcn_exp2f(m - m_use);  // 0 when m is -inf
+    l *= alpha;
+#pragma unroll
+    for (int dt = 0; dt < DT; dt++) o[dt] *= alpha;
+  }
+  l += rs;
+  m = m_new;
+  // P as f16 hi + lo, cells 32 j + 8 quad + e
+#pragma unroll
+  for (int j = 0; j < 2; j++)
+#pragma unroll
+    for (int e = 0; e < 8; e += 2) {
+      const f32x2 p = {st[2 * j + (e >> 2)][e & 3], st[2 * j + (e >> 2)][(e & 3) + 1]};
+      const f16x2 hi = __builtin_convertvector(p, f16x2);
+      const f32x2 r = {fmaf((float)hi[0], -1.0f, p[0]), fmaf((float)hi[1], -1.0f, p[1])};
+      const f16x2 lo = __builtin_convertvector(r, f16x2);
+      ph[j][e] = hi[0];
+      ph[j][e + 1] = hi[1];
+      pl[j][e] = lo[0];
+      pl[j][e + 1] = lo[1];
+    }
 }
 
 // Partial state of one (item, kv head): O^T rows then m, l per row.
@@ -230,8 +306,6 @@ paged_attn_kernel(const float *__restrict__ q, int H, int Hkv, float scale_log2,
   // half is zero in K and Q (the lanes of quads 2 and 3 load nothing)
   constexpr int KS = D >= 32 ? D / 32 : 1;
   constexpr int DT = D / 16;   // d tiles of the output
-  __shared__ __align__(16) uint16_t plh[ROWS * P_STRIDE];  // P as f16 hi
-  __shared__ __align__(16) uint16_t pll[ROWS * P_STRIDE];  // and lo
   __shared__ __align__(16) f16x8 qsh[KS * 64], qsl[KS * 64];  // Q fragments, hi and lo
 
   const int lane = threadIdx.x;
@@ -270,7 +344,7 @@ paged_attn_kernel(const float *__restrict__ q, int H, int Hkv, float scale_log2,
     for (int ct = 0; ct < 4; ct++)
 #pragma unroll
       for (int ks = 0; ks < KS; ks++)
-        kf[ct][ks] = kpart ? load_f16x8(kt + (ct * 16 + row) * D + ks * 32 + quad * 8)
+        kf[ct][ks] = kpart ? load_f16x8(kt + s_cell(ct, row) * D + ks * 32 + quad * 8)
                            : f16x8{0, 0, 0, 0, 0, 0, 0, 0};
   };
   auto load_v = [&](const uint16_t *vt) {
@@ -326,7 +400,10 @@ paged_attn_kernel(const float *__restrict__ q, int H, int Hkv, float scale_log2,
   // (straight-line code keeps the load counter waits exact, so the O
   // products do not wait for the next K). Heads of up to 128 run the last
   // block without NEXT, so no tile is loaded twice; heads of 256 (whose
-  // registers are full) load the last block's tiles again, from L2.
+  // registers are full) load the last block's tiles again, from L2
+  // (whose schedule is held in program order: left free, tiles in flight
+  // spilled, and a spill waits for them: 214 -> 260 us at 32 sequences of
+  // U[1024, 16384]).
   constexpr bool PEEL = D <= 128;
   auto block = [&](int blk, auto next) __attribute__((always_inline)) {
     constexpr bool NEXT = decltype(next)::value;
@@ -343,70 +420,19 @@ paged_attn_kernel(const float *__restrict__ q, int H, int Hkv, float scale_log2,
       }
       st[ct] = acc;
     }
+    if constexpr (!PEEL) __builtin_amdgcn_sched_barrier(0);
     if constexpr (NEXT) load_k(ktile(nxt));
 
-    // Mask and row max: lane holds cells ct*16 + quad*4 + i of its row. A
-    // block that ends at or before the group's first position (and, with a
+    // A block that ends at or before the group's first position (and, with a
     // window, starts inside the window of its last) is visible to every
     // valid row.
     const int cbase = blk * 64;
     const bool full = cbase + 63 <= p_first &&
                       (!RING || cbase > p_first + ntok - 1 - window);
-    float mx = -INFINITY;
-#pragma unroll
-    for (int ct = 0; ct < 4; ct++)
-#pragma unroll
-      for (int i = 0; i < 4; i++) {
-        const int p = cbase + ct * 16 + quad * 4 + i;
-        const bool vis = full || (p <= p_row && (!RING || p > p_row - window));
-        const float v = (rvalid && vis) ? st[ct][i] * scale_log2 : -INFINITY;
-        st[ct][i] = v;
-        mx = fmaxf(mx, v);
-      }
-    mx = fmaxf(mx, __shfl_xor(mx, 16));
-    mx = fmaxf(mx, __shfl_xor(mx, 32));
-    const float m_new = fmaxf(m, mx);
-    const float m_use = m_new == -INFINITY ? 0.0f : m_new;
-    float rs = 0.0f;
-#pragma unroll
-    for (int ct = 0; ct < 4; ct++) {
-      uint16_t ph[4], pq[4];
-#pragma unroll
-      for (int i = 0; i < 4; i++) {
-        const float pv = __builtin_amdgcn_exp2f(st[ct][i] - m_use);  // exp2(-inf) = 0
-        rs += pv;
-        const f16 hv = (f16)pv;
-        ph[i] = __builtin_bit_cast(uint16_t, hv);
-        pq[i] = f2h(pv - (float)hv);
-      }
-      const u32x2 wh = u32x2{(uint32_t)ph[0] | ((uint32_t)ph[1] << 16),
-                             (uint32_t)ph[2] | ((uint32_t)ph[3] << 16)};
-      const u32x2 wl = u32x2{(uint32_t)pq[0] | ((uint32_t)pq[1] << 16),
-                             (uint32_t)pq[2] | ((uint32_t)pq[3] << 16)};
-      *(u32x2 *)(plh + row * P_STRIDE + ct * 16 + quad * 4) = wh;
-      *(u32x2 *)(pll + row * P_STRIDE + ct * 16 + quad * 4) = wl;
-    }
-    rs += __shfl_xor(rs, 16);
-    rs += __shfl_xor(rs, 32);
-    // rescale only when some row's maximum moved
-    if (__builtin_amdgcn_ballot_w64(m_new != m)) {
-      const float alpha = __builtin_amdgcn_exp2f(m - m_use);  // 0 when m is -inf
-      l *= alpha;
-#pragma unroll
-      for (int dt = 0; dt < DT; dt++) o[dt] *= alpha;
-    }
-    l += rs;
-    m = m_new;
-    // The workgroup is one wave and a wave's LDS operations complete in
-    // order: a compiler barrier orders the P writes before the reads (an
-    // s_barrier would also wait for the next block's loads).
-    __asm__ volatile("" ::: "memory");
     f16x8 pfh[2], pfl[2];
-#pragma unroll
-    for (int kc = 0; kc < 2; kc++) {
-      pfh[kc] = load_f16x8(plh + row * P_STRIDE + kc * 32 + quad * 8);
-      pfl[kc] = load_f16x8(pll + row * P_STRIDE + kc * 32 + quad * 8);
-    }
+    softmax_block<DT>(st, scale_log2, full, cbase, quad, p_row, RING ? p_row - window + 1 : 0,
+                      rvalid, m, l, o, pfh, pfl);
+    if constexpr (!PEEL) __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int dt = 0; dt < DT; dt++)
 #pragma unroll
@@ -414,8 +440,8 @@ paged_attn_kernel(const float *__restrict__ q, int H, int Hkv, float scale_log2,
         o[dt] = mfma16(vf[dt][kc], pfh[kc], o[dt]);
         o[dt] = mfma16(vf[dt][kc], pfl[kc], o[dt]);
       }
+    if constexpr (!PEEL) __builtin_amdgcn_sched_barrier(0);
     if constexpr (NEXT) load_v(vtile(nxt));
-    __asm__ volatile("" ::: "memory");  // the P reads before the next block's writes
   };
   for (int blk = blo; blk + (PEEL ? 1 : 0) < bhi; blk++) block(blk, std::true_type{});
   if constexpr (PEEL)
@@ -441,8 +467,8 @@ paged_attn_kernel(const float *__restrict__ q, int H, int Hkv, float scale_log2,
 constexpr int SHARED_WAVES = ATTN_SHARED;
 
 template <int D>
-__device__ __forceinline__ int swk(int r) {
-  return D / 8 >= 16 ? (r & 15) : ((r >> 1) & 7);
+__device__ __forceinline__ int swk(int r) {  // distinct over the 16 rows of a tile (s_cell)
+  return D / 8 >= 16 ? (r & 3) | ((r >> 1) & 12) : ((r >> 1) & 1) | ((r >> 2) & 6);
 }
 __device__ __forceinline__ int swv(int r) { return (r >> 1) & 7; }
 
@@ -460,8 +486,6 @@ paged_attn_shared_kernel(const float *__restrict__ q, int H, int Hkv, float scal
   constexpr int KC = D / 8;                // 16-byte chunks per K row
   constexpr int LOADS = TILE / 8 / (64 * SHARED_WAVES);  // per lane and tile
   __shared__ __align__(16) uint16_t kb0[TILE], kb1[TILE], vb0[TILE], vb1[TILE];
-  __shared__ __align__(16) uint16_t plh_[SHARED_WAVES][ROWS * P_STRIDE];
-  __shared__ __align__(16) uint16_t pll_[SHARED_WAVES][ROWS * P_STRIDE];
   typedef __attribute__((address_space(3))) void lds_t;
 
   const int tid = threadIdx.x, lane = tid & 63;
@@ -477,7 +501,6 @@ paged_attn_shared_kernel(const float *__restrict__ q, int H, int Hkv, float scal
   const int tok0 = items[4 * item + 1];
   const int ntok = items[4 * item + 2] & 31;
   const int mg = (items[4 * item + 2] >> 5) - 1;
-  uint16_t *plh = plh_[wave], *pll = pll_[wave];
 
   const int row = lane & 15, quad = lane >> 4;
   const int rtok = row / G;
@@ -539,87 +562,58 @@ paged_attn_shared_kernel(const float *__restrict__ q, int H, int Hkv, float scal
     const int cbase = blk * 64;
     if (active && cbase <= p_last) {
       const uint16_t *kt = buf ? kb1 : kb0, *vt = buf ? vb1 : vb0;
-      // S^T[cell][row] for 4 tiles of 16 cells, K fragments from LDS
+      // S^T[cell][row] for 4 tiles of 16 cells; K fragments from LDS, the
+      // next step's read while one multiplies
       f32x4 st[4];
+      f16x8 kf[2][4];
+      auto read_k = [&](int ks, f16x8(&f)[4]) __attribute__((always_inline)) {
 #pragma unroll
-      for (int ct = 0; ct < 4; ct++) {
-        const int r = ct * 16 + row;
-        f16x8 kf[KS];
-#pragma unroll
-        for (int ks = 0; ks < KS; ks++)
-          kf[ks] = load_f16x8(kt + (r * KC + ((ks * 4 + quad) ^ swk<D>(r))) * 8);
-        f32x4 acc = f32x4{0, 0, 0, 0};
-#pragma unroll
-        for (int ks = 0; ks < KS; ks++) {
-          acc = mfma16(kf[ks], qh[ks], acc);
-          acc = mfma16(kf[ks], ql[ks], acc);
+        for (int ct = 0; ct < 4; ct++) {
+          const int r = s_cell(ct, row);
+          f[ct] = load_f16x8(kt + (r * KC + ((ks * 4 + quad) ^ swk<D>(r))) * 8);
         }
-        st[ct] = acc;
+      };
+      read_k(0, kf[0]);
+#pragma unroll
+      for (int ks = 0; ks < KS; ks++) {
+        if (ks + 1 < KS) read_k(ks + 1, kf[(ks + 1) & 1]);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int ct = 0; ct < 4; ct++)
+          st[ct] = mfma16(kf[ks & 1][ct], qh[ks], ks ? st[ct] : f32x4{0, 0, 0, 0});
+#pragma unroll
+        for (int ct = 0; ct < 4; ct++) st[ct] = mfma16(kf[ks & 1][ct], ql[ks], st[ct]);
+        __builtin_amdgcn_sched_barrier(0);
       }
-      const bool full = cbase + 63 <= p_first;
-      float mx = -INFINITY;
-#pragma unroll
-      for (int ct = 0; ct < 4; ct++)
-#pragma unroll
-        for (int i = 0; i < 4; i++) {
-          const int p = cbase + ct * 16 + quad * 4 + i;
-          const bool vis = full || p <= p_row;
-          const float v = (rvalid && vis) ? st[ct][i] * scale_log2 : -INFINITY;
-          st[ct][i] = v;
-          mx = fmaxf(mx, v);
-        }
-      mx = fmaxf(mx, __shfl_xor(mx, 16));
-      mx = fmaxf(mx, __shfl_xor(mx, 32));
-      const float m_new = fmaxf(m, mx);
-      const float m_use = m_new == -INFINITY ? 0.0f : m_new;
-      float rs = 0.0f;
-#pragma unroll
-      for (int ct = 0; ct < 4; ct++) {
-        uint16_t ph[4], pq[4];
-#pragma unroll
-        for (int i = 0; i < 4; i++) {
-          const float pv = __builtin_amdgcn_exp2f(st[ct][i] - m_use);  // exp2(-inf) = 0
-          rs += pv;
-          const f16 hv = (f16)pv;
-          ph[i] = __builtin_bit_cast(uint16_t, hv);
-          pq[i] = f2h(pv - (float)hv);
-        }
-        const u32x2 wh = u32x2{(uint32_t)ph[0] | ((uint32_t)ph[1] << 16),
-                               (uint32_t)ph[2] | ((uint32_t)ph[3] << 16)};
-        const u32x2 wl = u32x2{(uint32_t)pq[0] | ((uint32_t)pq[1] << 16),
-                               (uint32_t)pq[2] | ((uint32_t)pq[3] << 16)};
-        *(u32x2 *)(plh + row * P_STRIDE + ct * 16 + quad * 4) = wh;
-        *(u32x2 *)(pll + row * P_STRIDE + ct * 16 + quad * 4) = wl;
-      }
-      rs += __shfl_xor(rs, 16);
-      rs += __shfl_xor(rs, 32);
-      if (__builtin_amdgcn_ballot_w64(m_new != m)) {
-        const float alpha = __builtin_amdgcn_exp2f(m - m_use);  // 0 when m is -inf
-        l *= alpha;
-#pragma unroll
-        for (int dt = 0; dt < DT; dt++) o[dt] *= alpha;
-      }
-      l += rs;
-      m = m_new;
-      // a wave's LDS operations complete in order: the P writes before the reads
-      __asm__ volatile("" ::: "memory");
       f16x8 pfh[2], pfl[2];
+      softmax_block<DT>(st, scale_log2, cbase + 63 <= p_first, cbase, quad, p_row, 0, rvalid, m, l,
+                        o, pfh, pfl);
+      // O^T += V^T P^T, two d tiles at a time, the next two read meanwhile
+      f16x8 vf[2][2][2];
+      auto read_v = [&](int dt, f16x8(&f)[2][2]) __attribute__((always_inline)) {
 #pragma unroll
-      for (int kc = 0; kc < 2; kc++) {
-        pfh[kc] = load_f16x8(plh + row * P_STRIDE + kc * 32 + quad * 8);
-        pfl[kc] = load_f16x8(pll + row * P_STRIDE + kc * 32 + quad * 8);
-      }
+        for (int t = 0; t < 2; t++)
 #pragma unroll
-      for (int dt = 0; dt < DT; dt++) {
-        const int r = dt * 16 + row;
+          for (int kc = 0; kc < 2; kc++) {
+            const int r = (dt + t) * 16 + row;
+            f[t][kc] = load_f16x8(vt + (r * 8 + ((kc * 4 + quad) ^ swv(r))) * 8);
+          }
+      };
+      read_v(0, vf[0]);
+#pragma unroll
+      for (int dt = 0; dt < DT; dt += 2) {
+        const int b = dt >> 1 & 1;
+        if (dt + 2 < DT) read_v(dt + 2, vf[b ^ 1]);
+        __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (int kc = 0; kc < 2; kc++) {
-          const f16x8 vf = load_f16x8(vt + (r * 8 + ((kc * 4 + quad) ^ swv(r))) * 8);
-          o[dt] = mfma16(vf, pfh[kc], o[dt]);
-          o[dt] = mfma16(vf, pfl[kc], o[dt]);
+          o[dt] = mfma16(vf[b][0][kc], pfh[kc], o[dt]);
+          o[dt + 1] = mfma16(vf[b][1][kc], pfh[kc], o[dt + 1]);
+          o[dt] = mfma16(vf[b][0][kc], pfl[kc], o[dt]);
+          o[dt + 1] = mfma16(vf[b][1][kc], pfl[kc], o[dt + 1]);
         }
+        __builtin_amdgcn_sched_barrier(0);
       }
-      __asm__ volatile("" ::: "memory");  // the P reads before the next block's writes
     }
     __builtin_amdgcn_s_waitcnt(0);  // this wave's loads of blk + 1 have landed
     __syncthreads();                // ... and everyone's; buffer buf is free again
