@@ -210,6 +210,12 @@ struct Pending {
   }
 };
 
+// A workgroup barrier that waits for this wave's LDS operations only: global
+// loads stay in flight across it.
+__device__ __forceinline__ void lds_sync() {
+  asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+}
+
 // Cells per KV block; the pool layout and the attention tiles assume it.
 constexpr int KV_BLOCK = 64;
 // Query groups per shared attention run (lgmlh_plan's sets; the waves of

@@ -67,15 +67,6 @@ struct FlashArgs {
   float scale, max_bias, softcap;
 };
 
-// A workgroup barrier that waits for LDS operations only: global loads stay
-// in flight across it.
-__device__ __forceinline__ void fa_barrier() {
-  __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0)
-  asm volatile("" ::: "memory");
-  __builtin_amdgcn_s_barrier();
-  asm volatile("" ::: "memory");
-}
-
 // DP: the head size padded to the MFMA step (zeros past D); BC: cells per
 // tile.
 template <int DP, int BC, int RW, int KW>
@@ -423,7 +414,7 @@ __global__ void __launch_bounds__(RW *KW * 64, 1) flash_attn_kernel(FlashArgs A)
   // one wave needs no barrier: its LDS operations complete in order.
   auto turn_barrier = [&]() {
     if constexpr (KLDS)
-      fa_barrier();
+      lds_sync();
     else
       asm volatile("" ::: "memory");
   };
@@ -432,7 +423,7 @@ __global__ void __launch_bounds__(RW *KW * 64, 1) flash_attn_kernel(FlashArgs A)
   // tile's registers, loaded meanwhile, wait for the other: one barrier a
   // turn.
   const int turns = (ntiles + KW - 1) / KW;
-  fa_barrier();  // bad starts at zero
+  lds_sync();  // bad starts at zero
   u32x2 mc[CT];
   auto take_mask = [&]() {
 #pragma unroll
@@ -480,7 +471,7 @@ __global__ void __launch_bounds__(RW *KW * 64, 1) flash_attn_kernel(FlashArgs A)
     // the groups' states of a row tile, merged in group order
     float *const sl = (float *)lds;
     auto state = [&](int g) { return sl + (g * RW + rw) * 16 * (DP + 2); };
-    fa_barrier();
+    lds_sync();
     {
       float *s = state(kw);
 #pragma unroll
@@ -490,7 +481,7 @@ __global__ void __launch_bounds__(RW *KW * 64, 1) flash_attn_kernel(FlashArgs A)
         s[16 * DP + 16 + r16] = l;
       }
     }
-    fa_barrier();
+    lds_sync();
     if (kw != 0) return;
     float M = -INFINITY;
 #pragma unroll
