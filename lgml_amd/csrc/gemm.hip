@@ -318,10 +318,11 @@ struct WFrag<LGMLH_Q8_0> {
 // (C2's Q4_K shapes at N = 576: 4-15% faster, gate|up at N = 64 6%; the
 // mixed phase 3228 -> 3397 tok/s). Q6_K on ggml's X the same, with two X
 // buffers (70 KB): C2's Q6_K down products at a 512-token prefill pass 4.21
-// -> 3.27 ms. A tile's sums do not depend on the workgroup shape: each
+// -> 3.27 ms; and Q8_0 (78 KB): 2560 x 10240 at 512 rows 102 -> 92 us, 20480 x
+// 2560 172 -> 165. A tile's sums do not depend on the workgroup shape: each
 // 16-row tile takes the same fragments in the same K steps.
 __host__ __device__ constexpr int gemm_waves(int type, int nct, bool q8) {
-  return nct == 4 && (type == LGMLH_Q4_K || (type == LGMLH_Q6_K && q8)) ? 4 : GEMM_WAVES;
+  return nct == 4 && (type == LGMLH_Q4_K || q8) ? 4 : GEMM_WAVES;
 }
 //
 // Q8: X as ggml's quantized activations (split.h: Q8_K for Q4_K / Q6_K,
@@ -752,9 +753,9 @@ qgemm_kernel(const uint8_t *__restrict__ w, int64_t M, int64_t K, const f16 *__r
   float *const out = nz == 1 ? y : part + (int64_t)z * N * M;
   const int64_t ld_out = nz == 1 ? ldy : M;
   // The first split of a folded pair waits in part (y may be the
-  // residual). Compiled for the wide Q4_K / Q6_K tiles only: elsewhere the
-  // registers it holds would spill.
-  constexpr bool CAN_FOLD = NCT == 4 && !GATHER && TYPE != LGMLH_Q8_0;
+  // residual). Compiled for the wide tiles only, for Q8_0 in ggml's
+  // arithmetic: elsewhere the registers it holds would spill.
+  constexpr bool CAN_FOLD = NCT == 4 && !GATHER && (TYPE != LGMLH_Q8_0 || Q8);
   float *const pair = CAN_FOLD ? part + (int64_t)z * N * M : nullptr;
   // A lane's 4 values are consecutive rows of one output column: one
   // 16-byte store when the layout allows (4-byte stores spread over 16
@@ -1474,8 +1475,16 @@ static int launch_q(const void *w, int64_t M, int64_t K, const f16 *xs, int64_t 
   // consumers' reads of twice the partials (C2's 512-token prefill pass:
   // products 16.1 -> 15.2 ms, the rms_norm and rope consumers 1.85 ->
   // 2.29 ms, the pass 0.4 ms shorter than with pairs from 512 tiles).
-  const int fold =
-      splits > 1 && nct == 4 && TYPE != LGMLH_Q8_0 && tiles * splits >= 8192 ? SPLIT_PAIR : 1;
+  // A product of two splits whose sums nobody else adds (the plain entry
+  // points) runs them in one workgroup from 1024 workgroups up: no partial
+  // sums and no reduction launch (Q8_0 20480 x 2560 at 512 rows 165 -> 152 us,
+  // Q6_K 141 -> 123; with more splits the reduction stays and the pairs only
+  // make fewer rounds: Q4_K 4096 x 14336 at 575 rows 120 -> 128).
+  const bool can_fold = splits > 1 && nct == 4 && (TYPE != LGMLH_Q8_0 || Q8);
+  const int fold = can_fold && ((TYPE != LGMLH_Q8_0 && tiles * splits >= 8192) ||
+                                (!defer && splits == SPLIT_PAIR && tiles >= 1024))
+                       ? SPLIT_PAIR
+                       : 1;
   const int nz = (splits + fold - 1) / fold;
   *group = fold == 1 ? SPLIT_PAIR : 1;
   dim3 grid((unsigned)((N + cols - 1) / cols), (unsigned)((M + wrows - 1) / wrows),

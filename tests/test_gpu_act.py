@@ -122,6 +122,20 @@ def test_mul_mat_ggml_folded_pairs(L, ty):
     assert rel_err(y[rows], want) < 1e-5
 
 
+@pytest.mark.parametrize("ty", [core.Q4_K, core.Q6_K, core.Q8_0])
+def test_mul_mat_ggml_two_splits_in_one_workgroup(L, ty):
+    # two splits and 1024 workgroups (128 rows x 64 columns): no partial sums;
+    # 130 rows take the partial sums and the reduction, the same bits
+    M, K, N = 16384, 1024, 450
+    w = core.quantize(ty, core.fill_normal(M * K, 0, 0.02, 27).reshape(M, K))
+    x = act_rows(K, N, 28)
+    y = run_mul_mat_ggml(L, ty, w, M, K, x)
+    y130 = run_mul_mat_ggml(L, ty, w, M, K, x[:130])
+    assert np.array_equal(y[:130].view(np.uint32), y130.view(np.uint32))
+    rows = [0, 2, 130, N - 1]
+    assert rel_err(y[rows], core.mul_mat_q8(ty, w, M, K, x[rows])) < 1e-5
+
+
 def test_mul_mat_id_ggml(L):
     from lgml_amd import hip
     NE, M, K, T, U, nu = 16, 768, 2048, 40, 1, 8
