@@ -93,7 +93,7 @@ __global__ void __launch_bounds__(RW *KW * 64, 1) flash_attn_kernel(FlashArgs A)
   const int D = A.D, kvh = blockIdx.x;
   const int r16 = lane & 15, quad = lane >> 4;
   const int rows = A.T * A.G;
-  const int rr = (blockIdx.y * RW + rw) * 16 + r16;
+  const int rr = ((blockIdx.z * gridDim.y + blockIdx.y) * RW + rw) * 16 + r16;
   const bool rvalid = rr < rows;
   const int t = (rvalid ? rr : 0) / A.G, h = kvh * A.G + (rvalid ? rr : 0) % A.G;
   const float slope = alibi(h, A.H, A.max_bias);
@@ -129,10 +129,12 @@ __global__ void __launch_bounds__(RW *KW * 64, 1) flash_attn_kernel(FlashArgs A)
     }
     mx = fmaxf(mx, __shfl_xor(mx, 16));
     mx = fmaxf(mx, __shfl_xor(mx, 32));
-    // exponents of f32 normals; a zero, denormal or infinite maximum keeps 1
-    const int ex = (int)(__builtin_bit_cast(uint32_t, mx) >> 23);
+    // exponents of f32 normals (the largest take 2^-126: at most 4); a zero,
+    // denormal or infinite maximum keeps 1
+    int ex = (int)(__builtin_bit_cast(uint32_t, mx) >> 23);
     float inv = 1.0f;
-    if (ex > 1 && ex < 253) {
+    if (ex > 1 && ex < 255) {
+      ex = min(ex, 252);
       inv = __builtin_bit_cast(float, (uint32_t)(253 - ex) << 23);
       qscale = __builtin_bit_cast(float, (uint32_t)(ex + 1) << 23);
     }
@@ -513,9 +515,10 @@ __global__ void __launch_bounds__(RW *KW * 64, 1) flash_attn_kernel(FlashArgs A)
 
 template <int DP, int BC, int RW, int KW>
 static void launch_flash(const FlashArgs &A, int n_head_kv, hipStream_t st) {
-  const int64_t rows = (int64_t)A.T * A.G;
+  const int64_t tiles = ((int64_t)A.T * A.G + RW * 16 - 1) / (RW * 16);
+  const int64_t gy = tiles < 65535 ? tiles : 65535;  // the most a grid takes in y
   hipLaunchKernelGGL((flash_attn_kernel<DP, BC, RW, KW>),
-                     dim3((unsigned)n_head_kv, (unsigned)((rows + RW * 16 - 1) / (RW * 16))),
+                     dim3((unsigned)n_head_kv, (unsigned)gy, (unsigned)((tiles + gy - 1) / gy)),
                      dim3(RW * KW * 64), 0, st, A);
 }
 

@@ -221,3 +221,31 @@ def test_flash_attn_addresses_of_elements(L):
     got = out.cpu().numpy()
     assert got[0] == 0
     assert rel_err(got[1:].reshape(T * H, D), want.reshape(T * H, D)) < 1e-5
+
+
+def test_flash_attn_rows_near_the_largest_f32(L):
+    """q of up to 3.4e38 (past the exponents a power of two brings to 1)."""
+    rng = np.random.default_rng(62)
+    H, Hkv, T, D, n_kv = 2, 1, 5, 16, 40
+    q = rng.standard_normal((H, T, D)).astype(np.float32)
+    q[0] = np.sign(q[0]) * rng.uniform(0.5, 1.0, (T, D)).astype(np.float32) * np.float32(3.4e38)
+    k = core.f32_to_f16_bits(1e-3 * rng.standard_normal((Hkv, n_kv, D)).astype(np.float32))
+    v = core.f32_to_f16_bits(rng.standard_normal((Hkv, n_kv, D)).astype(np.float32))
+    m = core.f32_to_f16_bits(np.zeros((1, T, n_kv), np.float32))
+    got = gpu_flash(L, q, k, v, Hkv, n_kv, (D, n_kv * D), (D, n_kv * D), m, 0.25)
+    want = core.flash_attn(q, k, v, Hkv, m, 0.25, 0.0, 0.0)
+    assert rel_err(got.reshape(T * H, D), want.reshape(T * H, D)) < 1e-5
+
+
+def test_flash_attn_more_row_tiles_than_a_grid_has_in_y(L):
+    """65537 workgroups of 64 rows: the last ones write their rows too."""
+    from lgml_amd import hip
+    H, D = 8, 8
+    T = 65536 * 8 + 3
+    q = torch.ones(H * T * D, device="cuda")
+    k = torch.ones(D, dtype=torch.float16, device="cuda")
+    v = torch.arange(D, dtype=torch.float16, device="cuda")
+    out = torch.full((T * H, D), -1.0, device="cuda")
+    hip.check(L.lgmlh_flash_attn(q.data_ptr(), H, T, D, k.data_ptr(), v.data_ptr(), 1, 1, D, D, D,
+                                 D, 0, 1, T, 0.5, 0.0, 0.0, out.data_ptr(), st()))
+    assert bool((out == torch.arange(D, device="cuda").float()).all())
