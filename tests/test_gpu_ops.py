@@ -275,6 +275,29 @@ def test_get_rows(L, ty):
                             n, out.data_ptr(), st()) == hip.ERANGE
 
 
+@pytest.mark.parametrize("ty,cols,n", [
+    (core.F32, 1, 5), (core.F32, 1027, 3), (core.F16, 259, 9), (core.F16, 2, 300),
+    (core.Q8_0, 32, 1), (core.Q8_0, 1056, 6), (core.Q4_K, 256, 2), (core.Q6_K, 4352, 3)])
+def test_get_rows_ragged_columns(L, ty, cols, n):
+    """Columns that end inside a thread's four and inside a workgroup."""
+    from lgml_amd import hip
+    wf = core.fill_normal(11 * cols, 0, 0.5, 18).reshape(11, cols)
+    if ty in (core.F32, core.F16):
+        table = wf if ty == core.F32 else wf.astype(np.float16).view(np.uint16)
+        deq = wf if ty == core.F32 else wf.astype(np.float16).astype(np.float32)
+    else:
+        table = core.quantize(ty, wf)
+        deq = core.dequantize(ty, table, cols)
+    ids = (np.arange(n) * 7 % 11).astype(np.int32)
+    out = torch.full((n * cols + 4,), 9.0, dtype=torch.float32, device="cuda")
+    dt, dids = dev(table), dev(ids)
+    hip.check(L.lgmlh_get_rows(ty, dt.data_ptr(), 11, cols, dids.data_ptr(), ids.ctypes.data, n,
+                               out.data_ptr(), st()))
+    got = out.cpu().numpy()
+    assert (got[n * cols:] == 9.0).all()
+    assert np.array_equal(got[:n * cols].view(np.uint32), deq[ids].ravel().view(np.uint32))
+
+
 @pytest.mark.parametrize("case", [
     (core.F32, 64, 4096, 0.0, 0.02), (core.Q4_K, 256, 4096, 0.0, 0.02),
     (core.Q6_K, 128, 4096, 0.0, 0.02), (core.Q8_0, 160, 2560, 0.0, 0.02),
