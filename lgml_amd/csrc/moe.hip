@@ -331,6 +331,21 @@ __device__ void route_token(const float *__restrict__ part, int nz, int64_t T, i
 
 // ---- grouping of the picks by expert ------------------------------------------
 
+// The lanes of the wave whose pick is of this lane's expert e (e >= 0; all
+// lanes call it): a ballot per bit of the number, 9 steps where reading every
+// lane's e in turn took 64.
+__device__ __forceinline__ uint64_t same_expert(int e) {
+  static_assert(MOE_MAX_EXPERTS <= 512, "an expert's number is 9 bits");
+  uint64_t m = __builtin_amdgcn_ballot_w64(e >= 0);
+#pragma unroll
+  for (int b = 0; b < 9; b++) {
+    const bool on = (e >> b) & 1;
+    const uint64_t v = __builtin_amdgcn_ballot_w64(on);
+    m &= on ? v : ~v;
+  }
+  return m;
+}
+
 struct GroupLds {
   int32_t ids[MOE_MAX_PICKS];
   int32_t base[ROUTE_WAVES][MOE_MAX_EXPERTS];  // per wave chunk: counts, then bases
@@ -407,13 +422,8 @@ __device__ void group_picks(GroupLds &lds, int P, int NE, const GroupOut &go) {
   for (int r0 = lo; r0 < hi; r0 += 64) {
     const int p = r0 + lane;
     const int e = p < hi ? lds.ids[p] : -1;
-    int rank = 0, tot = 0;
-    for (int l2 = 0; l2 < 64; l2++) {
-      const int e2 = __builtin_amdgcn_readlane(e, l2);  // lane l2's expert, to every lane
-      const int same = e2 == e ? 1 : 0;
-      tot += same;
-      rank += l2 < lane ? same : 0;
-    }
+    const uint64_t same = same_expert(e);
+    const int rank = __popcll(same & ((1ull << lane) - 1)), tot = __popcll(same);
     const int b = e >= 0 ? lds.base[wave][e] : 0;
     if (e >= 0) go.sorted[b + rank] = p;
     __builtin_amdgcn_wave_barrier();  // all lanes read base before it moves
@@ -502,11 +512,7 @@ group_count_kernel(const int32_t *__restrict__ ids, int P, int NE, GroupOut go,
       for (int64_t m = 0; m < M; m++) y[(int64_t)p * M + m] = 0.0f;
   }
   // rank among the wave's earlier lanes with the same expert
-  int rank = 0;
-  for (int l2 = 0; l2 < 64; l2++) {
-    const int e2 = __builtin_amdgcn_readlane(e, l2);
-    rank += (l2 < lane && e2 == e) ? 1 : 0;
-  }
+  int rank = __popcll(same_expert(e) & ((1ull << lane) - 1));
   __syncthreads();
   if (e >= 0) atomicAdd(&cnt[wave][e], 1);  // counts: order-free
   __syncthreads();
@@ -532,18 +538,29 @@ group_place_kernel(int P, int NE, GroupOut go) {
   const int C = (P + GROUP_CHUNK - 1) / GROUP_CHUNK, c0 = blockIdx.x;
   // experts tid, tid + GROUP_CHUNK (NE <= 512): their totals and the picks
   // of the chunks before this one
-  constexpr int EPT = MOE_MAX_EXPERTS / GROUP_CHUNK;
+  constexpr int EPT = MOE_MAX_EXPERTS / GROUP_CHUNK, CB = 16;
+  const int p = c0 * GROUP_CHUNK + tid;
+  const int mine = p < P ? go.rank[p] : -1;
   int tot[EPT], pre[EPT];
 #pragma unroll
   for (int j = 0; j < EPT; j++) {
     const int e = tid + j * GROUP_CHUNK;
     tot[j] = pre[j] = 0;
-    if (e < NE)
-      for (int c = 0; c < C; c++) {
-        const int v = go.counts[(int64_t)c * NE + e];
-        tot[j] += v;
-        pre[j] += c < c0 ? v : 0;
+    if (j * GROUP_CHUNK >= NE) continue;
+    // CB chunks' counts in flight (chunks past C and experts past NE read
+    // the last one and add nothing)
+    const int32_t *src = go.counts + (e < NE ? e : NE - 1);
+    for (int c = 0; c < C; c += CB) {
+      int v[CB];
+#pragma unroll
+      for (int u = 0; u < CB; u++) v[u] = src[(int64_t)(c + u < C ? c + u : C - 1) * NE];
+#pragma unroll
+      for (int u = 0; u < CB; u++) {
+        const int x = c + u < C && e < NE ? v[u] : 0;
+        tot[j] += x;
+        pre[j] += c + u < c0 ? x : 0;
       }
+    }
   }
   // exclusive scans over the experts of the totals and of the tile counts:
   // expert e = tid + j GROUP_CHUNK, scanned in e order
@@ -587,11 +604,7 @@ group_place_kernel(int P, int NE, GroupOut go) {
     if (c0 == 0) *go.n_tiles = run_t;
   }
   __syncthreads();
-  const int p = c0 * GROUP_CHUNK + tid;
-  if (p < P) {
-    const int v = go.rank[p];
-    if (v >= 0) go.sorted[base[v >> 16] + (v & 0xffff)] = p;
-  }
+  if (mine >= 0) go.sorted[base[mine >> 16] + (mine & 0xffff)] = p;
   if (c0 != 0) return;
   // the tile list, expert by expert
   for (int e = tid; e < NE; e += GROUP_CHUNK) {

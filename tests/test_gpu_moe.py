@@ -126,6 +126,28 @@ def test_mul_mat_id_bad_ids_give_zero_rows(L):
     assert rel_err(got[mask], want[mask]) < 1e-5
 
 
+# One workgroup's grouping (to 1024 picks) and the chunked one past it: chunks of
+# 256 partly filled, 17 and 32 of them, 1 to 512 experts, numbers of no expert.
+@pytest.mark.parametrize("T,k,NE", [(1, 1, 1), (128, 8, 512), (129, 8, 512), (513, 8, 3),
+                                    (1024, 8, 300)])
+def test_picks_grouped_by_expert(L, T, k, NE):
+    M, K = 16, 256
+    rng = np.random.default_rng(T + NE)
+    wq = core.quantize(core.Q8_0, (rng.standard_normal((NE * M, K)) * 0.02).astype(np.float32))
+    w = core.dequantize(core.Q8_0, wq, K).reshape(NE, M, K)
+    x = rng.standard_normal((T, 1, K)).astype(np.float32)
+    ids = rng.integers(0, NE, size=(T, k)).astype(np.int32)
+    ids[T // 2:T // 2 + T // 8] = NE - 1  # whole waves of one expert
+    if T > 1:
+        ids[T - 1, 0], ids[0, k - 1], ids[3, 1] = -1, NE, -(1 << 31)
+    print("picks", T, k, NE, flush=True)
+    got = run_id(L, core.Q8_0, repacked_experts(L, core.Q8_0, wq, NE, M, K), NE, M, K, x, ids)
+    ok = (ids >= 0) & (ids < NE)
+    want = np.matmul(w[np.where(ok, ids, 0)].astype(np.float64), x[:, :, :, None])[..., 0]
+    assert not got[~ok].any()
+    assert rel_err(got[ok], want[ok]) < 1e-5
+
+
 def test_moe_sum(L):
     from lgml_amd import hip
     rng = np.random.default_rng(9)
