@@ -494,6 +494,9 @@ group_kernel(const int32_t *__restrict__ ids, int P, int NE, GroupOut go, float 
 // expert; group_place_kernel adds the counts of the chunks before its own
 // and the experts before each expert, and places its picks. The result is
 // the one-workgroup grouping's: expert-major, pick order within an expert.
+// Both are chains of latency: a wave's ranks by ballots and 16 chunks' counts in
+// flight at once took a layer of 512 x 8 picks over 128 experts (two groupings,
+// 4.9 + 7.0 us each before) 208.7 -> 200.5 us, one of 64 x 8 122.5 -> 118.9.
 constexpr int GROUP_CHUNK = 256;
 constexpr int GROUP_ONE = 1024;  // picks grouped by one workgroup
 
