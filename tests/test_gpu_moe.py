@@ -61,6 +61,33 @@ def test_route_matches_oracle(L, ne, k, gating, norm, scale, n):
     np.testing.assert_allclose(gw, ow, rtol=1e-6, atol=1e-7)
 
 
+@pytest.mark.parametrize("ne,k", [(5, 5), (16, 3), (128, 8), (300, 16), (512, 16)])
+def test_route_order_of_special_logits(L, ne, k):
+    """Ids are the logits in order, -0 equal to 0, ties to the smaller number,
+    infinities in their places; NaN is never picked (expert 0 once none is left)."""
+    from lgml_amd import hip
+    rng = np.random.default_rng(ne)
+    lg = rng.choice(np.array([0.0, -0.0, 1e-40, -1e-40, 1.5, -np.inf, np.inf, np.nan, -3.0],
+                             np.float32), (40, ne))
+    lg[0], lg[1], lg[2] = np.nan, -np.inf, -0.0
+    lg[2, ::2] = 0.0
+    lg[3, k - 2:] = np.nan
+    ids = torch.empty((40, k), dtype=torch.int32, device="cuda")
+    w = torch.empty((40, k), dtype=torch.float32, device="cuda")
+    lgd = dev(lg)
+    hip.check(L.lgmlh_moe_route(lgd.data_ptr(), 40, ne, k, hip.GATING_SIGMOID, 0, 1.0,
+                                ids.data_ptr(), w.data_ptr(), st()))
+    gi, gw = ids.cpu().numpy(), w.cpu().numpy()
+    for t in range(40):
+        want = sorted((e for e in range(ne) if lg[t, e] == lg[t, e]),
+                      key=lambda e: (-lg[t, e], e))[:k]
+        want += [0] * (k - len(want))
+        assert list(gi[t]) == want
+        with np.errstate(over="ignore"):
+            sig = 1 / (1 + np.exp(-lg[t, want].astype(np.float64)))
+        np.testing.assert_allclose(gw[t], sig, rtol=1e-6, atol=1e-7)
+
+
 def repacked_experts(L, ty, wq, NE, M, K):
     """n_expert matrices repacked back to back, as lgmlh_mul_mat_id takes them."""
     from lgml_amd import hip
