@@ -27,7 +27,7 @@
 // What bounds it: the f16 MFMAs (twice the products' flops for the hi + lo
 // pairs) and the softmax's VALU, which overlap only in part (the two waves of
 // a SIMD run in step). 32 / 8 heads of 128, 512 rows over 2048 cells under a
-// causal mask: 72.7 us, 207 TFLOP/s of the products (2460 us with one wave
+// causal mask: 66.2 us, 227 TFLOP/s of the products (2458 us with one wave
 // per query row and head, each column's dot product in VALU); without its
 // loads 56 us, without its products and softmax 27.
 #include <math.h>
