@@ -14,11 +14,16 @@
 // online softmax in f32 (a lane owns one row), and O^T += V^T P^T.
 //
 // K and V are exact f16; Q (scaled by a power of two to at most 1 per row,
-// so any f32 row fits f16) and P enter the MFMAs as f16 hi + lo pairs, so a
-// product is f32-accurate. The MFMA's k index over 32 cells is taken in the
-// order (quad, tile of 16, i): a lane's own S^T values then are its B operand
-// of the second product, with no trip through LDS, and V^T is stored in that
-// order of cells.
+// so any f32 row fits f16) and P enter the MFMAs as f16 hi + lo pairs. P is
+// held FA_P times as large (l and O with it, so that the factor cancels), and
+// its low parts are FA_LO times as large again, with products of their own:
+// a pair carries 22 bits of every P down to 2^-28, and what is lost below is
+// at most 2^-52 of the row's largest. (Unscaled, P below 2^-25 was 0 in O but
+// counted in l, and one cell 16 above 2048 others took 13% of the result;
+// P 2^15 times as large alone left 8e-6 there.) The MFMA's k index over 32
+// cells is taken in the order (quad, tile of 16, i): a lane's own S^T values
+// then are its B operand of the second product, with no trip through LDS, and
+// V^T is stored in that order of cells.
 //
 // A masked cell (mask -inf, or past n_kv) adds nothing whatever K and V
 // hold there: its score is set, and a V value that is not finite is stored
@@ -27,9 +32,9 @@
 // What bounds it: the f16 MFMAs (twice the products' flops for the hi + lo
 // pairs) and the softmax's VALU, which overlap only in part (the two waves of
 // a SIMD run in step). 32 / 8 heads of 128, 512 rows over 2048 cells under a
-// causal mask: 66.2 us, 227 TFLOP/s of the products (2458 us with one wave
-// per query row and head, each column's dot product in VALU); without its
-// loads 56 us, without its products and softmax 27.
+// causal mask: 69 us, 218 TFLOP/s of the products (2458 us with one wave per
+// query row and head, each column's dot product in VALU; 66 with P's low
+// parts unscaled and added in the MFMAs).
 #include <math.h>
 
 #include "common.h"
@@ -38,6 +43,7 @@ namespace lgmlh {
 
 constexpr int FA_MAX_D = 256;
 constexpr float FA_LOG2E = 1.4426950408889634f;
+constexpr float FA_P = 32768.0f, FA_LO = 4096.0f;  // the scales of P and of a low part
 
 // ALiBi slope of head h (1 without max_bias): with n the largest power of
 // two <= H, heads below n take (2^(-max_bias / n))^(h + 1), the others
@@ -331,7 +337,8 @@ __global__ void __launch_bounds__(RW *KW * 64, 1) flash_attn_kernel(FlashArgs A)
     for (int ct = 0; ct < CT; ct++)
 #pragma unroll
       for (int i = 0; i < 4; i++) {
-        st[ct][i] = __builtin_amdgcn_exp2f((st[ct][i] - m_use) * FA_LOG2E);  // exp2(-inf) = 0
+        // exp2(-inf) = 0
+        st[ct][i] = __builtin_amdgcn_exp2f((st[ct][i] - m_use) * FA_LOG2E) * FA_P;
         rs += st[ct][i];
       }
     rs += __shfl_xor(rs, 16);
@@ -351,7 +358,7 @@ __global__ void __launch_bounds__(RW *KW * 64, 1) flash_attn_kernel(FlashArgs A)
       for (int e = 0; e < 8; e += 2) {
         const f32x2 p = {st[2 * j + (e >> 2)][e & 3], st[2 * j + (e >> 2)][(e & 3) + 1]};
         const f16x2 hi = __builtin_convertvector(p, f16x2);
-        const f32x2 r = {fmaf((float)hi[0], -1.0f, p[0]), fmaf((float)hi[1], -1.0f, p[1])};
+        const f32x2 r = {(p[0] - (float)hi[0]) * FA_LO, (p[1] - (float)hi[1]) * FA_LO};
         const f16x2 lo = __builtin_convertvector(r, f16x2);
         ph[j][e] = hi[0];
         ph[j][e + 1] = hi[1];
@@ -364,9 +371,16 @@ __global__ void __launch_bounds__(RW *KW * 64, 1) flash_attn_kernel(FlashArgs A)
       for (int j = 0; j < CJ; j++)
         f[j] = *(const f16x8 *)(vl + (dt * 16 + r16) * VROW + j * 32 + quad * 8);
     };
-    // two tiles of D at a time, the next two read meanwhile
+    // two tiles of D at a time, the next two read meanwhile; their products
+    // with the low parts (FA_LO times too large) are added a turn later
     static_assert(DT % 2 == 0, "d tiles in pairs");
     f16x8 vg[2][CJ];
+    f32x4 lf[2], lg[2];
+    auto add_low = [&](int dt) {
+      const int b = dt >> 1 & 1;
+      o[dt] += lf[b] * (1.0f / FA_LO);
+      o[dt + 1] += lg[b] * (1.0f / FA_LO);
+    };
     read(0, vf[0]);
     read(1, vg[0]);
 #pragma unroll
@@ -379,13 +393,16 @@ __global__ void __launch_bounds__(RW *KW * 64, 1) flash_attn_kernel(FlashArgs A)
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
       for (int j = 0; j < CJ; j++) {
+        const f32x4 z = {0, 0, 0, 0};
         o[dt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vf[b][j], ph[j], o[dt], 0, 0, 0);
         o[dt + 1] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vg[b][j], ph[j], o[dt + 1], 0, 0, 0);
-        o[dt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vf[b][j], pl[j], o[dt], 0, 0, 0);
-        o[dt + 1] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vg[b][j], pl[j], o[dt + 1], 0, 0, 0);
+        lf[b] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vf[b][j], pl[j], j ? lf[b] : z, 0, 0, 0);
+        lg[b] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vg[b][j], pl[j], j ? lg[b] : z, 0, 0, 0);
       }
+      if (dt > 0) add_low(dt - 2);
       __builtin_amdgcn_sched_barrier(0);
     }
+    add_low(DT - 2);
     // V values that are not finite, to the rows that see their cells
     for (int w = 0; w < 2; w++) {
       uint32_t b = __builtin_amdgcn_readfirstlane(bad[it % 3][kw][w]);

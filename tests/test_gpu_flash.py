@@ -140,9 +140,9 @@ def test_flash_attn_on_pool_rows_equals_paged_attention(L):
 # share them, rows around 16 and 64 (the last two cases: from 96 workgroups
 # of 64 rows, four row tiles each), head sizes that are and are not whole
 # MFMA steps. The bound is the one of the other cases: hi + lo pairs carry 22
-# bits, so products and their f32 sums over up to 256 + 300 terms stay within
-# 556 * 2^-24 + 2^-21 of the largest term, 3.4e-5; errors add at random and
-# measure 4e-7.
+# bits of these scores and probabilities, so products and their f32 sums over
+# up to 256 + 300 terms stay within 556 * 2^-24 + 2^-21 of the largest term,
+# 3.4e-5; errors add at random and measure 4e-7.
 EDGES = [  # H, Hkv, T, D, n_kv
     (1, 1, 1, 8, 1), (3, 1, 5, 16, 31), (2, 2, 16, 40, 32), (4, 1, 4, 64, 33), (4, 2, 9, 96, 63),
     (2, 1, 8, 128, 64), (8, 2, 1, 128, 65), (2, 1, 3, 160, 129), (2, 2, 17, 192, 255),
@@ -199,6 +199,44 @@ def test_flash_attn_masked_cells_hold_anything(L, T):
     assert np.isinf(got[sees[:, 0], 0, 7]).all() and np.isfinite(got[1]).all()
     got[:, :2, 7], clean[:, :2, 7] = 0, 0
     assert rel_err(got.reshape(T * H, D), clean.reshape(T * H, D)) < 1e-5
+
+
+def softmax64(s, v):
+    """Rows of softmax(s) v in f64 (s (rows, cells), v (cells, D))."""
+    p = np.exp(s - s.max(axis=1, keepdims=True))
+    return p @ v.astype(np.float64) / p.sum(axis=1, keepdims=True)
+
+
+# One cell that takes almost all of a row's weight, above thousands of others
+# whose sum is the result (the cell's V is 0) or a part of it. Scores are
+# exact (one value of q and k), so a row loses: its argument of exp2, |s|
+# log2(e) <= 26, rounded to f32 (2^-20 ln 2 = 6.6e-7) with log2(e) itself
+# (2e-7), P's 22 bits and exp2's last bit (2.4e-7 each), and a rounding of l and
+# O per turn (16 rows: 8 groups of 32 cells; 1024 rows: 2 groups of 64). The
+# sums are alike from row to row, so the roundings may all go one way. It
+# measures a third to a half of the bound.
+@pytest.mark.parametrize("n_kv", [2048, 32768])
+@pytest.mark.parametrize("T", [16, 1024])
+@pytest.mark.parametrize("sink_v", [0, 1])
+def test_flash_attn_one_cell_above_thousands(L, n_kv, T, sink_v):
+    rng = np.random.default_rng(63)
+    H, Hkv, D = 8, 8, 32
+    gaps = np.linspace(1, 16, T).astype(np.float16).astype(np.float32)  # a gap per row
+    q = np.zeros((H, T, D), np.float32)
+    q[:, :, 3] = gaps
+    k = np.zeros((n_kv, Hkv, D), np.float16)
+    k[5, :, 3] = 1.0
+    k[7::7, :, 3] = -0.125
+    v = rng.standard_normal((n_kv, Hkv, D)).astype(np.float16)
+    v[5] *= sink_v
+    got = gpu_flash(L, q, k.view(np.uint16), v.view(np.uint16), Hkv, n_kv, (Hkv * D, D),
+                    (Hkv * D, D), None, 1.0)
+    for h in range(H):
+        want = softmax64(gaps[:, None].astype(np.float64) * k[None, :, h, 3].astype(np.float64),
+                         v[:, h])
+        err = np.linalg.norm(got[:, h] - want, axis=1) / np.linalg.norm(want, axis=1)
+        turns = n_kv // (32 * 8 if T == 16 else 64 * 2)
+        assert err.max() < 1.4e-6 + turns * 2.0 ** -23, (h, gaps[err.argmax()], err.max())
 
 
 def test_flash_attn_addresses_of_elements(L):
