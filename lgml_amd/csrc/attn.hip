@@ -10,10 +10,16 @@
 // (K rows straight from the [cell][D] tile), an online softmax per row in
 // f32 (each lane owns one row; reductions over 4 lanes with shuffles), and
 // O^T += V^T P^T (V columns straight from the transposed [D][cell] tile, P
-// from the lane's own S^T values: s_cell). K and V are exact f16; Q and P enter the MFMAs as
-// f16 hi + lo pairs, so every product is f32-accurate. The loads of block
-// b + 1 are issued as soon as block b's registers are consumed (K after
-// S, V after O), so they overlap block b's softmax and products.
+// from the lane's own S^T values: s_cell). K and V are exact f16; Q and P
+// enter the MFMAs as f16 hi + lo pairs, P held ATTN_P times as large (l and O
+// with it: the factor cancels), so that a pair carries 22 bits of every P down
+// to 2^-17 of the row's largest, and below is at most 2^-40 of that off.
+// (Unscaled, P below 2^-25 was 0 in O but counted in l: one cell 16 above 2000
+// others made 4% to 20% of the result wrong. 64 decoding sequences of 32 / 8
+// heads of 128 take 106 us either way, a 512-token chunk beside 32 sequences
+// 163 and 164.) The loads of block b + 1 are issued as soon as block b's
+// registers are consumed (K after S, V after O), so they overlap block b's
+// softmax and products.
 // Items start longest run first (the plan's order): all of a launch's
 // waves are resident at once, and the ones that share a SIMD with an older
 // wave advance slowly until it ends, so those should be the shortest.
@@ -35,6 +41,7 @@ namespace lgmlh {
 
 constexpr int ROWS = 16;      // MFMA rows per wave
 constexpr float LOG2E = 1.4426950408889634f;
+constexpr float ATTN_P = 32768.0f;  // the scale of P
 
 __device__ __forceinline__ f32x4 mfma16(f16x8 a, f16x8 b, f32x4 c) {
   return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0);
@@ -91,7 +98,7 @@ __device__ __forceinline__ void softmax_block(f32x4 (&st)[4], float scale_log2, 
   for (int ct = 0; ct < 4; ct++)
 #pragma unroll
     for (int i = 0; i < 4; i++) {
-      st[ct][i] = __builtin_amdgcn_exp2f(st[ct][i] - m_use);  // exp2(-inf) = 0
+      st[ct][i] = __builtin_amdgcn_exp2f(st[ct][i] - m_use) * ATTN_P;  // exp2(-inf) = 0
       rs += st[ct][i];
     }
   rs += __shfl_xor(rs, 16);

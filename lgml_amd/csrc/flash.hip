@@ -19,8 +19,8 @@
 // its low parts are FA_LO times as large again, with products of their own:
 // a pair carries 22 bits of every P down to 2^-28, and what is lost below is
 // at most 2^-52 of the row's largest. (Unscaled, P below 2^-25 was 0 in O but
-// counted in l, and one cell 16 above 2048 others took 13% of the result;
-// P 2^15 times as large alone left 8e-6 there.) The MFMA's k index over 32
+// counted in l, and one cell 16 above 2048 others made 4% to 20% of the
+// result wrong; P 2^15 times as large alone leaves up to 8e-6 there.) The MFMA's k index over 32
 // cells is taken in the order (quad, tile of 16, i): a lane's own S^T values
 // then are its B operand of the second product, with no trip through LDS, and
 // V^T is stored in that order of cells.

@@ -368,6 +368,42 @@ def test_paged_attention_order_changes_no_bits(L, H, Hkv, D):
         assert np.array_equal(a.view(np.uint32), b.view(np.uint32)), bps
 
 
+@pytest.mark.parametrize("H,Hkv,D", [(4, 2, 64), (8, 4, 128), (4, 2, 256)])
+def test_paged_attention_one_cell_above_thousands(L, H, Hkv, D):
+    """A cell (its V zero) that takes almost all of a row's weight, by 1 to 16
+    nats, above two thousand others whose sum is the result: a decode token
+    and a prompt chunk. A row loses its argument of exp2 rounded to f32 (8.7e-7 at
+    16 nats), P's 22 bits and exp2's last bit (2.4e-7 each), a rounding of l
+    and of O per 64-cell block (32 of them, possibly all one way), and P's grain
+    of 2^-40 beside p = exp(-gap)."""
+    seqs = [(1, 2000), (80, 1900)]
+    n_cells = 8192
+    _, kpool, vpool, bt = make_attn_case(H, Hkv, D, seqs, seed=91)
+    rng = np.random.default_rng(92)
+    k = np.zeros((n_cells, Hkv, D), np.float16)
+    v = rng.standard_normal((n_cells, Hkv, D)).astype(np.float16)
+    for i in range(2):
+        k[bt[i, 0] * 64 + 5, :, 3] = 1.0
+        v[bt[i, 0] * 64 + 5] = 0
+    N = 81
+    gaps = np.concatenate([[16.0], np.linspace(1, 16, 80)])
+    q = np.zeros((N, H, D), np.float32)
+    q[:, :, 3] = (gaps * np.sqrt(D))[:, None]
+    got, plan = gpu_attention(L, q, k.reshape(n_cells, -1).view(np.uint16),
+                              v.reshape(n_cells, -1).view(np.uint16), H, Hkv, D, seqs, bt)
+    assert plan.info.n_single > 0 and (D > 128 or plan.info.n_shared > 0)
+    for t in range(N):
+        i, past = (0, 2000) if t == 0 else (1, 1900 + t - 1)
+        pos = np.arange(past + 1)
+        cells = bt[i, pos // 64].astype(np.int64) * 64 + pos % 64
+        gap = float(q[t, 0, 3]) * float(np.float32(1 / np.sqrt(D)))
+        p = np.where(pos == 5, 1.0, np.exp(-gap))
+        for h in range(H):
+            want = p @ v[cells, h // (H // Hkv)].astype(np.float64) / p.sum()
+            err = np.linalg.norm(got[t, h] - want) / np.linalg.norm(want)
+            assert err < 1.4e-6 + 32 * 2.0 ** -23 + np.exp(gap) * 2.0 ** -40, (t, h, gap, err)
+
+
 def test_plan_cells_and_errors(L):
     from lgml_amd import hip, runtime
     from oracle import kvpool as kp
