@@ -13,12 +13,15 @@
 // was computed; a wave computes S^T = K Q^T with 16x16x32 f16 MFMAs, an
 // online softmax in f32 (a lane owns one row), and O^T += V^T P^T.
 //
-// K and V are exact f16; Q (scaled by a power of two to at most 1 per row,
-// so any f32 row fits f16) and P enter the MFMAs as f16 hi + lo pairs. P is
-// held FA_P times as large (l and O with it, so that the factor cancels), and
-// its low parts are FA_LO times as large again, with products of their own:
-// a pair carries 22 bits of every P down to 2^-28, and what is lost below is
-// at most 2^-52 of the row's largest. (Unscaled, P below 2^-25 was 0 in O but
+// K and V are exact f16; Q and P enter the MFMAs as f16 hi + lo pairs, with
+// the largest of a row near f16's (Q by a power of two per row, so any f32
+// row fits; P is held FA_P times as large, l and O with it, so that the
+// factor cancels) and the low parts FA_LO times as large again, with products
+// of their own: a pair carries 22 bits of every value down to 2^-28 of the
+// row's largest, and what is lost below is at most 2^-51 of that. (With the
+// largest at 1 and one sum for both, q values below 2^-14 of it lost bits: rows
+// with one value 2^14 to 2^22 times the others, where K is 0, were wrong by up
+// to 24%. P below 2^-25 was 0 in O but
 // counted in l, and one cell 16 above 2048 others made 4% to 20% of the
 // result wrong; P 2^15 times as large alone leaves up to 8e-6 there.) The MFMA's k index over 32
 // cells is taken in the order (quad, tile of 16, i): a lane's own S^T values
@@ -110,10 +113,10 @@ __global__ void __launch_bounds__(RW *KW * 64, 1) flash_attn_kernel(FlashArgs A)
 
   if (threadIdx.x < 6 * KW) (&bad[0][0][0])[threadIdx.x] = 0;
 
-  // Q fragments: row rr scaled by 2^-e (e the exponent of its largest |q|),
-  // hi + lo.
+  // Q fragments: row rr scaled by a power of two that brings its largest |q| to
+  // [2^14, 2^15), hi + lo.
   f16x8 qh[KS], ql[KS];
-  float qscale = 1.0f;
+  float qscale;
   {
     const float *qr = A.q + ((int64_t)h * A.T + t) * D;
     float x[KS][8], mx = 0.0f;
@@ -135,22 +138,17 @@ __global__ void __launch_bounds__(RW *KW * 64, 1) flash_attn_kernel(FlashArgs A)
     }
     mx = fmaxf(mx, __shfl_xor(mx, 16));
     mx = fmaxf(mx, __shfl_xor(mx, 32));
-    // exponents of f32 normals (the largest take 2^-126: at most 4); a zero,
-    // denormal or infinite maximum keeps 1
-    int ex = (int)(__builtin_bit_cast(uint32_t, mx) >> 23);
-    float inv = 1.0f;
-    if (ex > 1 && ex < 255) {
-      ex = min(ex, 252);
-      inv = __builtin_bit_cast(float, (uint32_t)(253 - ex) << 23);
-      qscale = __builtin_bit_cast(float, (uint32_t)(ex + 1) << 23);
-    }
+    // (rows below 2^-112 by the power of that)
+    const int ex = min(max((int)(__builtin_bit_cast(uint32_t, mx) >> 23), 15), 254);
+    const float inv = __builtin_bit_cast(float, (uint32_t)(268 - ex) << 23);
+    qscale = __builtin_bit_cast(float, (uint32_t)(ex - 14) << 23);
 #pragma unroll
     for (int ks = 0; ks < KS; ks++)
 #pragma unroll
       for (int e = 0; e < 8; e++) {
         const float v = x[ks][e] * inv;
         qh[ks][e] = (f16)v;
-        ql[ks][e] = (f16)(v - (float)qh[ks][e]);
+        ql[ks][e] = (f16)((v - (float)qh[ks][e]) * FA_LO);
       }
   }
   // with a softcap the scale goes inside the tanh: softcap tanh(s (scale / softcap))
@@ -280,6 +278,8 @@ __global__ void __launch_bounds__(RW *KW * 64, 1) flash_attn_kernel(FlashArgs A)
         f[ct] = KLDS ? *(const f16x8 *)(kl + (ct * 16 + r16) * KROW + ks * 32 + quad * 8)
                      : __builtin_bit_cast(f16x8, kr[(ct * KS + ks) % KU]);
     };
+    f32x4 low[CT];  // FA_LO times the products with the low parts
+    const f32x4 z = {0, 0, 0, 0};
     read(0, kf[0]);
 #pragma unroll
     for (int ks = 0; ks < KS; ks++) {
@@ -287,13 +287,14 @@ __global__ void __launch_bounds__(RW *KW * 64, 1) flash_attn_kernel(FlashArgs A)
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
       for (int ct = 0; ct < CT; ct++)
-        st[ct] = __builtin_amdgcn_mfma_f32_16x16x32_f16(
-            kf[ks & 1][ct], qh[ks], ks ? st[ct] : f32x4{0, 0, 0, 0}, 0, 0, 0);
+        st[ct] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kf[ks & 1][ct], qh[ks], ks ? st[ct] : z, 0, 0, 0);
 #pragma unroll
       for (int ct = 0; ct < CT; ct++)
-        st[ct] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kf[ks & 1][ct], ql[ks], st[ct], 0, 0, 0);
+        low[ct] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kf[ks & 1][ct], ql[ks], ks ? low[ct] : z, 0, 0, 0);
       __builtin_amdgcn_sched_barrier(0);
     }
+#pragma unroll
+    for (int ct = 0; ct < CT; ct++) st[ct] += low[ct] * (1.0f / FA_LO);
   };
   // The softmax of a tile (its mask values in mc) and its products with V.
   auto compute = [&](int tile, int it, const uint16_t *vl, const u32x2 (&mc)[CT]) {

@@ -239,6 +239,29 @@ def test_flash_attn_one_cell_above_thousands(L, n_kv, T, sink_v):
         assert err.max() < 1.4e-6 + turns * 2.0 ** -23, (h, gaps[err.argmax()], err.max())
 
 
+@pytest.mark.parametrize("T", [3, 500])
+@pytest.mark.parametrize("size", [1.0, 1e-36, 1e30])
+def test_flash_attn_one_value_of_q_far_above_the_others(L, T, size):
+    """Rows of q whose largest value meets zeros in K: the others, 2^-14 to
+    2^-22 of it, make the scores, and pairs hold 22 bits of them. With D = 64
+    products and sums of up to 200 terms the bound is that of the tile edges;
+    rows far from 1 in size are scaled the same way."""
+    rng = np.random.default_rng(64)
+    H, Hkv, D, n_kv = 16, 8, 64, 200
+    q = rng.standard_normal((H, T, D)).astype(np.float32)
+    q[:, :, 3] = 2.0 ** rng.integers(14, 23, (H, T))
+    k = rng.standard_normal((n_kv, Hkv, D)).astype(np.float16)
+    k[:, :, 3] = 0
+    v = rng.standard_normal((n_kv, Hkv, D)).astype(np.float16)
+    q = (q * np.float32(size)).astype(np.float32)
+    scale = float(np.float32(0.125 / size))
+    got = gpu_flash(L, q, k.view(np.uint16), v.view(np.uint16), Hkv, n_kv, (Hkv * D, D),
+                    (Hkv * D, D), None, scale)
+    for h in range(H):
+        s = q[h].astype(np.float64) @ k[:, h // 2].astype(np.float64).T * scale
+        assert rel_err(got[:, h], softmax64(s, v[:, h // 2])) < 1e-5, h
+
+
 def test_flash_attn_addresses_of_elements(L):
     """q, v, the mask and out start at any element (k is 16-byte aligned)."""
     from lgml_amd import hip
