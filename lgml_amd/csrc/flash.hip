@@ -21,12 +21,19 @@
 // row's largest, and what is lost below is at most 2^-51 of that. (With the
 // largest at 1 and one sum for both, q values below 2^-14 of it lost bits: rows
 // with one value 2^14 to 2^22 times the others, where K is 0, were wrong by up
-// to 24%. P below 2^-25 was 0 in O but
-// counted in l, and one cell 16 above 2048 others made 4% to 20% of the
-// result wrong; P 2^15 times as large alone leaves up to 8e-6 there.) The MFMA's k index over 32
-// cells is taken in the order (quad, tile of 16, i): a lane's own S^T values
-// then are its B operand of the second product, with no trip through LDS, and
-// V^T is stored in that order of cells.
+// to 24%. P below 2^-25 was 0 in O but counted in l, and one cell 16 above
+// 2048 others made 4% to 20% of the result wrong; P 2^15 times as large alone
+// leaves up to 8e-6 there.) The MFMA's k index over 32 cells is taken in the
+// order (quad, tile of 16, i): a lane's own S^T values then are its B operand
+// of the second product, with no trip through LDS, and V^T is stored in that
+// order of cells.
+//
+// An infinity in Q or K has no pair: its products with the low parts are NaN
+// where the score is an infinity (-inf drops the cell; with a softcap it is
+// one of +- softcap). A row that ends with a sum that is not a number is
+// therefore computed again from f32 products (exact_row), whichever it holds.
+// (At the end it costs other calls up to 1.5%; scoring the tile again where it
+// happens took registers of the loop, 512 x 2048 cells 69 -> 72 us.)
 //
 // A masked cell (mask -inf, or past n_kv) adds nothing whatever K and V
 // hold there: its score is set, and a V value that is not finite is stored
@@ -75,6 +82,59 @@ struct FlashArgs {
   int64_t k_rs, k_hs, v_rs, v_hs;
   float scale, max_bias, softcap;
 };
+
+// Row rr of KV head kvh by one wave, from f32 products: a cell per lane, then
+// D / 64 output values per lane.
+__device__ void exact_row(const FlashArgs &A, int kvh, int rr) {
+  const int t = rr / A.G, h = kvh * A.G + rr % A.G, lane = threadIdx.x & 63;
+  const float slope = alibi(h, A.H, A.max_bias);
+  const float *qr = A.q + ((int64_t)h * A.T + t) * A.D;
+  const uint16_t *mr = A.mask ? A.mask + ((int64_t)(h % A.mask_heads) * A.mask_rows + t) * A.n_kv
+                              : nullptr;
+  const uint16_t *kb = A.k + (int64_t)kvh * A.k_hs, *vb = A.v + (int64_t)kvh * A.v_hs;
+  const float sc = A.softcap > 0.0f ? A.scale / A.softcap : A.scale;
+  float m = -INFINITY, l = 0.0f, o[FA_MAX_D / 64];
+#pragma unroll
+  for (int i = 0; i < FA_MAX_D / 64; i++) o[i] = 0.0f;
+  for (int j0 = 0; j0 < A.n_kv; j0 += 64) {
+    const int j = j0 + lane;
+    const float mv = j >= A.n_kv ? -INFINITY : mr ? h2f(mr[j]) : 0.0f;
+    float s = -INFINITY;
+    if (mv != -INFINITY) {
+      float a = 0.0f;
+#pragma unroll 1
+      for (int d = 0; d < A.D; d++) a = fmaf(qr[d], h2f(kb[(int64_t)j * A.k_rs + d]), a);
+      a *= sc;
+      if (A.softcap > 0.0f) a = A.softcap * tanhf(a);
+      s = a + slope * mv;
+    }
+    float mt = s;
+    for (int x = 32; x > 0; x >>= 1) mt = fmaxf(mt, __shfl_xor(mt, x));
+    const float mn = fmaxf(m, mt), mu = mn == -INFINITY ? 0.0f : mn;
+    const float corr = expf(m - mu), p = expf(s - mu);  // 0 at -inf
+    float ps = p;
+    for (int x = 32; x > 0; x >>= 1) ps += __shfl_xor(ps, x);
+    l = l * corr + ps;
+#pragma unroll
+    for (int i = 0; i < FA_MAX_D / 64; i++) o[i] *= corr;
+    const int nj = min(A.n_kv - j0, 64);
+#pragma unroll 1
+    for (int jj = 0; jj < nj; jj++) {
+      const float pj = __shfl(p, jj);
+      if (pj == 0.0f) continue;  // wave-uniform
+      const uint16_t *vr = vb + (int64_t)(j0 + jj) * A.v_rs;
+#pragma unroll
+      for (int i = 0; i < FA_MAX_D / 64; i++)
+        if (lane + 64 * i < A.D) o[i] = fmaf(pj, h2f(vr[lane + 64 * i]), o[i]);
+    }
+    m = mn;
+  }
+  float *orow = A.out + ((int64_t)t * A.H + h) * A.D;
+  const float inv = l == 0.0f ? 0.0f : 1.0f / l;
+#pragma unroll
+  for (int i = 0; i < FA_MAX_D / 64; i++)
+    if (lane + 64 * i < A.D) orow[lane + 64 * i] = o[i] * inv;
+}
 
 // DP: the head size padded to the MFMA step (zeros past D); BC: cells per
 // tile.
@@ -519,16 +579,21 @@ __global__ void __launch_bounds__(RW *KW * 64, 1) flash_attn_kernel(FlashArgs A)
       for (int dt = 0; dt < DT; dt++) o[dt] += *(const f32x4 *)(s + (dt * 64 + lane) * 4) * w;
     }
   }
-  if (!rvalid) return;
-  // a row with every cell masked gives zeros
-  const float inv = l == 0.0f ? 0.0f : 1.0f / l;
-  float *orow = A.out + ((int64_t)t * A.H + h) * D;
+  if (rvalid && l == l) {
+    // a row with every cell masked gives zeros
+    const float inv = l == 0.0f ? 0.0f : 1.0f / l;
+    float *orow = A.out + ((int64_t)t * A.H + h) * D;
 #pragma unroll
-  for (int dt = 0; dt < DT; dt++) {
-    const int d0 = dt * 16 + quad * 4;
-    if (d0 >= D) continue;
-    *(f32x4_u *)(orow + d0) = o[dt] * inv;
+    for (int dt = 0; dt < DT; dt++) {
+      const int d0 = dt * 16 + quad * 4;
+      if (d0 >= D) continue;
+      *(f32x4_u *)(orow + d0) = o[dt] * inv;
+    }
   }
+  uint32_t lost = (uint32_t)__builtin_amdgcn_ballot_w64(rvalid && l != l) & 0xffffu;
+#pragma unroll 1
+  for (; lost; lost &= lost - 1)
+    exact_row(A, kvh, ((blockIdx.z * gridDim.y + blockIdx.y) * RW + rw) * 16 + __builtin_ctz(lost));
 }
 
 template <int DP, int BC, int RW, int KW>

@@ -262,6 +262,44 @@ def test_flash_attn_one_value_of_q_far_above_the_others(L, T, size):
         assert rel_err(got[:, h], softmax64(s, v[:, h // 2])) < 1e-5, h
 
 
+@pytest.mark.parametrize("softcap", [0.0, 20.0])
+@pytest.mark.parametrize("T,D", [(3, 64), (500, 64), (4, 128), (400, 128), (3, 256)])
+def test_flash_attn_seen_infinities_in_q_and_k(L, T, D, softcap):
+    """A score of -inf drops its cell, one of +inf or NaN makes its row NaN;
+    with a softcap infinite scores are +- softcap. K holds infinities that
+    rows see (q with and without a low part, or 0, beside them), and so does q."""
+    rng = np.random.default_rng(65)
+    H, Hkv, n_kv = 16, 8, 150
+    q = rng.standard_normal((H, T, D)).astype(np.float32)
+    q[:, :, 3:5] = np.abs(q[:, :, 3:5])
+    q[3::4] = q[3::4].astype(np.float16)
+    q[2, :, 3] *= -1        # +inf at cell 5
+    q[4, 0, 4] = 0          # 0 * inf at cell 77
+    q[5, 1, 7] = np.inf     # K is below 0 there: no cell left
+    q[7, 2, 8] = -np.inf    # and of both signs here
+    k = rng.standard_normal((n_kv, Hkv, D)).astype(np.float16)
+    k[:, :, 7] = -np.abs(k[:, :, 7])
+    k[5, :, 3] = -np.inf
+    k[77, :, 4] = -np.inf
+    k[130, 6] = np.nan
+    v = rng.standard_normal((n_kv, Hkv, D)).astype(np.float16)
+    got = gpu_flash(L, q, k.view(np.uint16), v.view(np.uint16), Hkv, n_kv, (Hkv * D, D),
+                    (Hkv * D, D), None, D ** -0.5, 0.0, softcap)
+    n_nan = 0
+    with np.errstate(invalid="ignore"):
+        for h in range(H):
+            s = (q[h].astype(np.float64)[:, None] * k[None, :, h // 2].astype(np.float64)).sum(2)
+            s = s * D ** -0.5
+            s = softcap * np.tanh(s / softcap) if softcap else s
+            want = softmax64(s, v[:, h // 2])
+            want[s.max(axis=1) == -np.inf] = 0  # no cell left
+            bad = np.isnan(want).any(axis=1)
+            assert np.isnan(got[bad, h]).all() and np.isfinite(got[~bad, h]).all(), h
+            assert not (~bad).any() or rel_err(got[~bad, h], want[~bad]) < 1e-5, h
+            n_nan += int(bad.sum())
+    assert 2 * T < n_nan < 4 * T  # heads 12 and 13, which see the NaN, and single rows
+
+
 def test_flash_attn_addresses_of_elements(L):
     """q, v, the mask and out start at any element (k is 16-byte aligned)."""
     from lgml_amd import hip
