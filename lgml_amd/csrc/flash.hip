@@ -85,8 +85,8 @@ struct FlashArgs {
 
 // Row rr of KV head kvh by one wave, from f32 products: a cell per lane, then
 // D / 64 output values per lane.
-__device__ void exact_row(const FlashArgs &A, int kvh, int rr) {
-  const int t = rr / A.G, h = kvh * A.G + rr % A.G, lane = threadIdx.x & 63;
+__device__ void exact_row(const FlashArgs &A, int kvh, uint32_t rr) {
+  const int t = rr / (uint32_t)A.G, h = kvh * A.G + rr % (uint32_t)A.G, lane = threadIdx.x & 63;
   const float slope = alibi(h, A.H, A.max_bias);
   const float *qr = A.q + ((int64_t)h * A.T + t) * A.D;
   const uint16_t *mr = A.mask ? A.mask + ((int64_t)(h % A.mask_heads) * A.mask_rows + t) * A.n_kv
@@ -161,10 +161,11 @@ __global__ void __launch_bounds__(RW *KW * 64, 1) flash_attn_kernel(FlashArgs A)
   auto kl_of = [&](int it) { return stage0 + (NB == 2 ? (it & 1) * (KT + VT) : 0); };
   const int D = A.D, kvh = blockIdx.x;
   const int r16 = lane & 15, quad = lane >> 4;
-  const int rows = A.T * A.G;
-  const int rr = ((blockIdx.z * gridDim.y + blockIdx.y) * RW + rw) * 16 + r16;
+  // (rows past 2^31 fit a GPU: 32-bit, but unsigned)
+  const uint32_t G = A.G, rows = A.T * G;
+  const uint32_t rr = ((blockIdx.z * gridDim.y + blockIdx.y) * RW + rw) * 16 + r16;
   const bool rvalid = rr < rows;
-  const int t = (rvalid ? rr : 0) / A.G, h = kvh * A.G + (rvalid ? rr : 0) % A.G;
+  const int t = (rvalid ? rr : 0) / G, h = kvh * A.G + (rvalid ? rr : 0) % G;
   const float slope = alibi(h, A.H, A.max_bias);
   const uint16_t *mr = A.mask ? A.mask + ((int64_t)(h % A.mask_heads) * A.mask_rows + t) * A.n_kv
                               : nullptr;

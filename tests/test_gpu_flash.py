@@ -348,3 +348,22 @@ def test_flash_attn_more_row_tiles_than_a_grid_has_in_y(L):
     hip.check(L.lgmlh_flash_attn(q.data_ptr(), H, T, D, k.data_ptr(), v.data_ptr(), 1, 1, D, D, D,
                                  D, 0, 1, T, 0.5, 0.0, 0.0, out.data_ptr(), st()))
     assert bool((out == torch.arange(D, device="cuda").float()).all())
+
+
+def test_flash_attn_more_rows_than_an_int_counts(L):
+    """2^31 + 192 (token, query head) pairs of one KV head."""
+    from lgml_amd import hip
+    H, D, T = 64, 8, 2 ** 25 + 3
+    if torch.cuda.mem_get_info()[0] < 2 * H * T * D * 4 + (8 << 30):
+        pytest.skip("needs 137 GB")
+    q = torch.ones(H * T * D, device="cuda")
+    k = torch.ones(D, dtype=torch.float16, device="cuda")
+    v = torch.arange(1, D + 1, dtype=torch.float16, device="cuda")
+    out = torch.zeros(T * H, D, device="cuda")
+    hip.check(L.lgmlh_flash_attn(q.data_ptr(), H, T, D, k.data_ptr(), v.data_ptr(), 1, 1, D, D, D,
+                                 D, 0, 1, T, 0.5, 0.0, 0.0, out.data_ptr(), st()))
+    want = torch.arange(1, D + 1, device="cuda").float()
+    for at in (0, 2 ** 30, 2 ** 31 - 4096, T * H - 4096):
+        assert bool((out[at:at + 4096] == want).all()), at
+    del q, out
+    torch.cuda.empty_cache()
