@@ -211,7 +211,7 @@ static size_t ws_bytes_of(const Sizes &z) {
     add((size_t)router_splits(z.E) * z.N * z.NE * 4);  // router partials
     add(z.P * 4);                                        // ids
     add(z.P * 4);                                        // weights
-    add(group_bytes(z.P, z.NE, z.tc));                   // grouping
+    add(group_bytes(z.P, z.NE));                   // grouping
     add(z.P * 2 * z.FX * 4);                             // [gate | up] of the picks
     add(z.P * z.FX * 4);                                 // f32 activations (f32 experts)
     add(z.P * z.E * 4);                                  // expert outputs (pending)
@@ -378,7 +378,7 @@ extern "C" int lgmlh_forward(const lgmlh_model *m, const lgmlh_ubatch *ub,
     rpart = (float *)cv.take((size_t)router_splits(z.E) * z.N * z.NE * 4);
     mids = (int32_t *)cv.take(z.P * 4);
     mwts = (float *)cv.take(z.P * 4);
-    void *gb = cv.take(group_bytes(z.P, z.NE, z.tc));
+    void *gb = cv.take(group_bytes(z.P, z.NE));
     gu_e = (float *)cv.take(z.P * 2 * z.FX * 4);
     act_e = (float *)cv.take(z.P * z.FX * 4);
     y_e = (float *)cv.take(z.P * z.E * 4);

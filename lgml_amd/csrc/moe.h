@@ -23,7 +23,7 @@ int router_logits(const float *w, int NE, int64_t K, const float *x, int64_t T, 
 int moe_route_dev(const float *part, int nz, int64_t T, int NE, int n_used, int gating,
                   int norm_topk, float scale, int32_t *ids, float *wts, const GroupOut *go,
                   hipStream_t st);
-size_t group_bytes(int64_t P, int NE, int tc);
+size_t group_bytes(int64_t P, int NE);
 GroupOut group_carve(void *ws, int64_t P, int NE, int tc);
 int experts_dev(int type, const void *w, int NE, int64_t M, int64_t K, const float *xf,
                 const f16 *xs, int64_t xnpad, int U, const int32_t *ids, int64_t T, int n_used,

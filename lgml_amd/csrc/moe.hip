@@ -768,12 +768,18 @@ int moe_route_dev(const float *part, int nz, int64_t T, int NE, int n_used, int 
 }
 
 // Workspace of a grouping of P picks: sorted, tiles, count, and the
-// many-workgroup grouping's ranks and chunk counts.
+// many-workgroup grouping's ranks and chunk counts. The tile list has room for
+// 16-column tiles at any P (never fewer than 64-column ones), so that the size
+// never falls as P grows and a workspace made for the largest batch holds
+// every smaller one, on either side of the switch to 64 columns.
+static size_t tiles_bytes(int64_t P, int NE) {
+  return a256((size_t)moe_max_tiles(P, NE, 16) * 16);
+}
 static int64_t group_chunks(int64_t P) { return (P + GROUP_CHUNK - 1) / GROUP_CHUNK; }
 
-size_t group_bytes(int64_t P, int NE, int tc) {
-  return a256((size_t)P * 4) + a256((size_t)moe_max_tiles(P, NE, tc) * 16) + 256 +
-         a256((size_t)P * 4) + a256((size_t)group_chunks(P) * NE * 4);
+size_t group_bytes(int64_t P, int NE) {
+  return a256((size_t)P * 4) + tiles_bytes(P, NE) + 256 + a256((size_t)P * 4) +
+         a256((size_t)group_chunks(P) * NE * 4);
 }
 
 GroupOut group_carve(void *ws, int64_t P, int NE, int tc) {
@@ -782,7 +788,7 @@ GroupOut group_carve(void *ws, int64_t P, int NE, int tc) {
   g.sorted = (int32_t *)b;
   b += a256((size_t)P * 4);
   g.tiles = (int4 *)b;
-  b += a256((size_t)moe_max_tiles(P, NE, tc) * 16);
+  b += tiles_bytes(P, NE);
   g.n_tiles = (int32_t *)b;
   b += 256;
   g.rank = (int32_t *)b;
@@ -847,8 +853,7 @@ extern "C" size_t lgmlh_mul_mat_id_workspace(int type, int64_t n_expert, int64_t
                                              int64_t T, int64_t U, int n_used) {
   (void)M;
   const int64_t P = T * n_used;
-  const int tc = moe_tile_cols(P, (int)n_expert);
-  size_t b = group_bytes(P, (int)n_expert, tc);
+  size_t b = group_bytes(P, (int)n_expert);
   if (type != LGMLH_F32) b += a256(split_bytes(T * U, K));
   return b;
 }
@@ -891,7 +896,7 @@ static int mul_mat_id_entry(int act, int type, const void *w, int64_t n_expert, 
   f16 *xs = nullptr;
   const int xform = xf_for(type, act);
   if (type != LGMLH_F32) {
-    xs = (f16 *)((char *)workspace + group_bytes(P, NE, tc));
+    xs = (f16 *)((char *)workspace + group_bytes(P, NE));
     LGMLH_TRY(split_x(x, xtype, T * U, K, xs, st, xform));
   }
   return experts_dev(type, w, NE, M, K, (const float *)x, xs, split_npad(T * U), (int)U, ids, T,

@@ -94,6 +94,19 @@ def test_moe_entry_points_check_arguments(hip):
     assert L.lgmlh_moe_route(dummy, 4, 4, 8, 1, 1, 1.0, dummy, dummy, None) == hip.EINVAL
 
 
+@pytest.mark.parametrize("ne,used", [(1, 1), (8, 2), (8, 8), (32, 4), (32, 8), (64, 6), (128, 8),
+                                     (256, 8), (512, 16)])
+def test_mul_mat_id_workspace_never_falls_as_rows_grow(hip, ne, used):
+    """A workspace made for a caller's largest batch holds every smaller one."""
+    L = hip.lib()
+    for ty in (hip.Q4_K, hip.Q8_0, hip.F32):
+        for u in (1, used):
+            size = [L.lgmlh_mul_mat_id_workspace(ty, ne, 512, 256, t, u, used)
+                    for t in range(8192 // used + 1)]
+            falls = [t for t in range(1, len(size)) if size[t] < size[t - 1]]
+            assert not falls, (ty, u, falls)
+
+
 def test_sizes(hip):
     L = hip.lib()
     assert L.lgmlh_row_size(hip.Q4_K, 4096) == 16 * 144
