@@ -155,7 +155,12 @@ static Sizes sizes_of(const lgmlh_model *m, int64_t n_tokens, int64_t n_items, i
   z.NU = z.moe ? m->n_used : 0;
   z.FX = z.moe ? m->n_ff_exp : 0;
   z.P = z.N * z.NU;
-  z.tc = z.moe ? moe_tile_cols(z.P, z.NE) : 16;
+  // one grouping for a layer's two products (of 2 FX and E rows)
+  int exp_type = LGMLH_Q8_0;
+  for (int il = 0; il < m->n_layer; il++)
+    if (m->layers[il].gate_inp && m->layers[il].exp_gu_type != LGMLH_Q8_0)
+      exp_type = m->layers[il].exp_gu_type;
+  z.tc = z.moe ? moe_tile_cols(exp_type, 2 * z.FX < z.E ? 2 * z.FX : z.E, z.P, z.NE) : 16;
   for (int il = 0; il < m->n_layer; il++) {
     const lgmlh_layer &L = m->layers[il];
     const LDims d = dims_of(m, L);

@@ -15,7 +15,7 @@ struct GroupOut {
   int32_t *counts;    // [chunks][NE] scratch of the many-workgroup grouping
 };
 
-int moe_tile_cols(int64_t P, int NE);
+int moe_tile_cols(int type, int64_t M, int64_t P, int NE);
 int moe_max_tiles(int64_t P, int NE, int tc);
 int router_splits(int64_t K);
 int router_logits(const float *w, int NE, int64_t K, const float *x, int64_t T, float *part,

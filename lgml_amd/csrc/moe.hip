@@ -666,18 +666,30 @@ __global__ void moe_sum_kernel(const float *__restrict__ y, const float *__restr
 // ---- host side --------------------------------------------------------------------
 static size_t a256(size_t b) { return (b + 255) & ~size_t(255); }
 
-// Column tile width for P picks over NE experts: 64 once an expert averages
-// 24 picks and there are 1024 of them (or it averages 128), else 16. A
-// 64-column tile works on its 16-column parts in use, so it builds an
-// expert's weight fragments once where 16-column tiles build them per 16
-// picks; 16-column ones run twice the waves per CU. (The MoE layer of 512 x 8
-// picks over 128 experts of 768 x 2048, 32 picks each: Q4_K 262 us in 16-
-// column tiles, 222 in 64-column ones, Q8_0 387 and 286; 16 picks each: 169
-// and 175; 8 experts with 32 picks each, too few tiles to fill the chip: 58
-// and 67.)
-int moe_tile_cols(int64_t P, int NE) {
+// Column tile width of the products of M rows with P picks over NE experts: 64
+// or 16. A 64-column tile works on its 16-column parts in use, so it builds an
+// expert's weight fragments once where 16-column tiles build them per 16 picks;
+// 16-column ones make more workgroups and run twice the waves per CU. So 64
+// columns from 24 picks per expert, 1024 in all and 320 workgroups up (Q8_0,
+// whose weights are the most bytes, from 256 at 32 picks), and from 128
+// picks. The MoE layer in us, 16-column tiles / 64-column ones, embedding x
+// width of an expert, picks in all:
+//   128 experts 2048 x 768, 4096: Q4_K 229 / 198, Q8_0 375 / 276; 2048 (16
+//     each): the first 156, and 169 / 175 before the parts were left out
+//   64 of 2048 x 768, 1536: Q4_K 117 / 111; 4096: 205 / 175, Q8_0 352 / 243
+//   32 of 2048 x 768, 1024: 100 / 84; 2048, of which half the second tiles are
+//     nearly empty: 135 / 130 (f32-accurate 149 / 157); 3072: 170 / 142
+//   32 of 1280 x 768, 1536 (320 workgroups): 94 / 84, Q8_0 125 / 98
+//   32 of 1024 x 512, 1536 (256): 69 / 74, Q8_0 89 / 84
+//   64 of 512 x 256, 3072 (256): 61 / 67, Q8_0 74 / 72; 4096 (384): 70.6 / 69.3
+int moe_tile_cols(int type, int64_t M, int64_t P, int NE) {
   const int64_t ne = NE;
-  return P >= 128 * ne || (P >= 24 * ne && P >= 1024) ? 64 : 16;
+  if (P >= 128 * ne) return 64;
+  if (P < 24 * ne || P < 1024) return 16;
+  // about a tile per expert, past 56 picks each a second one for some
+  const int64_t tiles = P < 56 * ne ? ne : P / 64 + ne / 2;
+  const int64_t wgs = tiles * ((M + 127) / 128);
+  return wgs >= (type == LGMLH_Q8_0 && P >= 32 * ne ? 256 : 320) ? 64 : 16;
 }
 
 // An upper bound of the tiles of a grouping: sum over experts of
@@ -889,7 +901,7 @@ static int mul_mat_id_entry(int act, int type, const void *w, int64_t n_expert, 
   if (P == 0) return LGMLH_OK;
   hipStream_t st = as_stream(stream);
   const int NE = (int)n_expert;
-  const int tc = moe_tile_cols(P, NE);
+  const int tc = moe_tile_cols(type, M, P, NE);
   GroupOut go = group_carve(workspace, P, NE, tc);
   launch_group(ids, (int)P, NE, go, y, M, st);
   LGMLH_TRY(hip_check(hipGetLastError(), "mul_mat_id group"));

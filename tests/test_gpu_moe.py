@@ -227,13 +227,13 @@ def test_c5_batched_pass_equals_lone_pass():
 @pytest.mark.parametrize("ggml", [False, True])
 def test_grouped_product_tile_parts(ty, ggml):
     """64-column tiles with every number of 16-column parts in use: experts
-    with 0, 1, 15 .. 17, 31 .. 33, 47 .. 49, 63 .. 65 and more picks (1024
-    picks in all, so that the wide tiles run)."""
+    with 0, 1, 15 .. 17, 31 .. 33, 47 .. 49, 63 .. 65 and more picks (128
+    picks per expert on average, so that the wide tiles run)."""
     from lgml_amd import hip
     L = hip.lib()
     counts = [0, 1, 15, 16, 17, 31, 32, 33, 47, 48, 49, 63, 64, 65, 128, 129, 200]
     NE, M, K, nu = len(counts) + 2, 80, 512, 1
-    T = 2100
+    T = 2500
     ids = np.concatenate([np.full(n, e) for e, n in enumerate(counts)])
     ids = np.concatenate([ids, np.full((T - len(ids)) // 2, NE - 2)])
     ids = np.concatenate([ids, np.full(T - len(ids), NE - 1)]).astype(np.int32)
@@ -258,3 +258,43 @@ def test_grouped_product_tile_parts(ty, ggml):
                  y.data_ptr(), ws.data_ptr(), n, stream))
     want = core.mul_mat_id(ty, w, NE, M, K, x, ids, act_quant=ggml)
     assert rel_err(y.cpu().numpy().reshape(T, M), want.reshape(T, M)) < 1e-5
+
+
+@pytest.mark.parametrize("ty", [core.Q4_K, core.Q8_0])
+@pytest.mark.parametrize("ggml", [False, True])
+@pytest.mark.parametrize("M", [1024, 1152, 1280])
+def test_grouped_product_on_both_sides_of_the_tile_rule(ty, ggml, M):
+    """1024 picks over 32 experts: M = 1024, 1152 and 1280 rows make 256, 288
+    and 320 workgroups of 64-column tiles, around the numbers from which they
+    run. A row of the call gives the same bits in a call of its own (16-column
+    tiles)."""
+    from lgml_amd import hip
+    L = hip.lib()
+    NE, K, nu, T = 32, 256, 8, 128
+    rng = np.random.default_rng(M)
+    ids = np.stack([rng.permutation(NE)[:nu] for _ in range(T)]).astype(np.int32)
+    w = core.quantize(ty, core.fill_normal(NE * M * K, 0, 0.02, 33).reshape(NE * M, K))
+    x = core.fill_normal(T * K, 0, 1, 34).reshape(T, 1, K)
+    eb = L.lgmlh_repacked_bytes(ty, M, K)
+    rp = torch.empty(NE * eb, dtype=torch.uint8, device="cuda")
+    stream = torch.cuda.current_stream().cuda_stream
+    for e in range(NE):
+        src = torch.from_numpy(w[e * M:(e + 1) * M].copy()).cuda()
+        hip.check(L.lgmlh_repack(ty, M, K, src.data_ptr(), rp.data_ptr() + e * eb, stream))
+        torch.cuda.synchronize()
+    n = L.lgmlh_mul_mat_id_workspace(ty, NE, M, K, T, 1, nu)
+    ws = torch.empty(n, dtype=torch.uint8, device="cuda")
+    xd, idd = torch.from_numpy(x).cuda(), torch.from_numpy(ids).cuda()
+    fn = L.lgmlh_mul_mat_id_ggml if ggml else L.lgmlh_mul_mat_id
+
+    def run(lo, hi):
+        y = torch.empty((hi - lo, nu, M), device="cuda")
+        hip.check(fn(ty, rp.data_ptr(), NE, M, K, xd[lo:hi].data_ptr(), hip.F32, 1,
+                     idd[lo:hi].data_ptr(), hi - lo, nu, y.data_ptr(), ws.data_ptr(), n, stream))
+        return y
+
+    y = run(0, T)
+    want = core.mul_mat_id(ty, w, NE, M, K, x[:4], ids[:4], act_quant=ggml)
+    assert rel_err(y[:4].cpu().numpy().reshape(4 * nu, M), want.reshape(4 * nu, M)) < 1e-5
+    for t in (0, 77, T - 1):
+        assert torch.equal(run(t, t + 1)[0], y[t])
