@@ -23,18 +23,28 @@ typedef f32x4 f32x4_u __attribute__((aligned(4)));
 namespace lgmlh {
 
 // The launch of an elementwise kernel over n rows of `per_row` threads each:
-// threads along the row in whole waves (blocks of up to 256, several short
-// rows to a block), rows in blockIdx.y and threadIdx.y; a grid of at most
-// 65535 in y, past which the kernel's row loop goes on.
+// threads along the row in whole waves, several short rows to a block, a
+// row per thread (row_of), rows past a grid's 65535 in y in its z. Blocks are of
+// ROW_BLOCK threads, and the kernels say so in their launch bounds: without,
+// they are compiled for 1024, at most 128 registers, and a loop over rows
+// instead of z took swiglu_split_kernel past that (51 spilled, 152 bytes of
+// scratch a lane: 512 rows of 14336 27.6 us, 18.6 so) and get_rows_kernel and
+// splitk_reduce_kernel from 8 waves per SIMD to 4 (512 rows of 4096 12.8 and
+// 9.3 us; two splits of 512 x 20480 22.3 and 18.7).
+constexpr int ROW_BLOCK = 256;
 struct RowGrid {
   dim3 grid, block;
   RowGrid(int64_t per_row, int64_t n) {
     const int64_t bx = per_row > 128 ? 256 : per_row > 64 ? 128 : 64;
-    const int64_t by = 256 / bx, gy = (n + by - 1) / by;
+    const int64_t by = ROW_BLOCK / bx, tiles = n > 0 ? (n + by - 1) / by : 1;
+    const int64_t gy = tiles < 65535 ? tiles : 65535;
     block = dim3((unsigned)bx, (unsigned)by);
-    grid = dim3((unsigned)((per_row + bx - 1) / bx), (unsigned)(gy < 65535 ? gy : 65535));
+    grid = dim3((unsigned)((per_row + bx - 1) / bx), (unsigned)gy, (unsigned)((tiles + gy - 1) / gy));
   }
 };
+__device__ __forceinline__ int64_t row_of() {
+  return ((int64_t)blockIdx.z * gridDim.y + blockIdx.y) * blockDim.y + threadIdx.y;
+}
 
 // Thread-local error text behind lgmlh_last_error().
 void set_error(const char *fmt, ...);

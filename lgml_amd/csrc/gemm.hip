@@ -1246,54 +1246,51 @@ qstream_kernel(const uint8_t *__restrict__ w, int64_t M, int64_t K, const f16 *_
 // The partial sums of a split-K product, added in the canonical order
 // (Pending::sum): pairs of splits, then the pairs in order, then the
 // residual.
-__global__ void splitk_reduce_kernel(Pending pd, float *__restrict__ y, int64_t ldy,
-                                     const float *__restrict__ residual) {
+__global__ void __launch_bounds__(ROW_BLOCK)
+splitk_reduce_kernel(Pending pd, float *__restrict__ y, int64_t ldy,
+                     const float *__restrict__ residual) {
   const int64_t M = pd.cols, m = 4 * (blockIdx.x * (int64_t)blockDim.x + threadIdx.x);
-  if (m >= M) return;
+  const int64_t n = row_of();
+  if (m >= M || n >= pd.rows) return;
   const bool vec = (M & 3) == 0;  // 4 columns a thread; rows of partials then start at 16 bytes
-  for (int64_t n = blockIdx.y * (int64_t)blockDim.y + threadIdx.y; n < pd.rows;
-       n += (int64_t)gridDim.y * blockDim.y) {
-    float *yr = y + n * ldy + m;
-    const float *rr = residual ? residual + n * ldy + m : nullptr;
-    if (vec) {
-      float v[4];
-      pd.sum4(n, m, v);
-      f32x4 o = {v[0], v[1], v[2], v[3]};
-      if (rr) o += *(const f32x4_u *)rr;
-      *(f32x4_u *)yr = o;
-    } else {
-      for (int e = 0; e < 4 && m + e < M; e++) {
-        const float v = pd.sum(n, m + e);
-        yr[e] = rr ? v + rr[e] : v;
-      }
+  float *yr = y + n * ldy + m;
+  const float *rr = residual ? residual + n * ldy + m : nullptr;
+  if (vec) {
+    float v[4];
+    pd.sum4(n, m, v);
+    f32x4 o = {v[0], v[1], v[2], v[3]};
+    if (rr) o += *(const f32x4_u *)rr;
+    *(f32x4_u *)yr = o;
+  } else {
+    for (int e = 0; e < 4 && m + e < M; e++) {
+      const float v = pd.sum(n, m + e);
+      yr[e] = rr ? v + rr[e] : v;
     }
   }
 }
 
 // X (f32 or f16 rows of K) -> planes of the form xf; one thread per 8 values
 // (the lanes of a 256-value block are consecutive and leave together).
-__global__ void xsplit_kernel(const void *__restrict__ x, int xtype, int64_t N, int64_t K,
-                              f16 *__restrict__ planes, int64_t Npad, int xf) {
-  const int64_t k0 = 8 * (blockIdx.x * (int64_t)blockDim.x + threadIdx.x);
-  if (k0 >= K) return;  // K % 256 == 0: whole blocks of lanes leave together
-  for (int64_t n = blockIdx.y * (int64_t)blockDim.y + threadIdx.y; n < N;
-       n += (int64_t)gridDim.y * blockDim.y) {
-    float v[8];
-    if (xtype == LGMLH_F32) {
-      const f32x4 *p = (const f32x4 *)((const float *)x + n * K + k0);
-      f32x4 a = p[0], b = p[1];
+__global__ void __launch_bounds__(ROW_BLOCK)
+xsplit_kernel(const void *__restrict__ x, int xtype, int64_t N, int64_t K,
+              f16 *__restrict__ planes, int64_t Npad, int xf) {
+  const int64_t k0 = 8 * (blockIdx.x * (int64_t)blockDim.x + threadIdx.x), n = row_of();
+  if (k0 >= K || n >= N) return;  // K % 256 == 0: whole blocks of lanes leave together
+  float v[8];
+  if (xtype == LGMLH_F32) {
+    const f32x4 *p = (const f32x4 *)((const float *)x + n * K + k0);
+    f32x4 a = p[0], b = p[1];
 #pragma unroll
-      for (int e = 0; e < 4; e++) {
-        v[e] = a[e];
-        v[4 + e] = b[e];
-      }
-    } else {
-      f16x8 h = *(const f16x8 *)((const f16 *)x + n * K + k0);
-#pragma unroll
-      for (int e = 0; e < 8; e++) v[e] = (float)h[e];
+    for (int e = 0; e < 4; e++) {
+      v[e] = a[e];
+      v[4 + e] = b[e];
     }
-    act_store8(xf, planes, Npad, K, n, k0, v);
+  } else {
+    f16x8 h = *(const f16x8 *)((const f16 *)x + n * K + k0);
+#pragma unroll
+    for (int e = 0; e < 8; e++) v[e] = (float)h[e];
   }
+  act_store8(xf, planes, Npad, K, n, k0, v);
 }
 
 // ---- f32 weights: 16x16x4 f32 MFMAs ---------------------------------------------

@@ -631,34 +631,31 @@ f32_id_kernel(const float *__restrict__ w, int NE, int64_t M, int64_t K,
 // out[t][m] = (y[t][0][m] w[t][0] + y[t][1][m] w[t][1] + ...) (+ residual),
 // products and sums in pick order (g:mul then sum_picks).
 // Four columns a thread, the picks' values of eight picks in flight.
-__global__ void moe_sum_kernel(const float *__restrict__ y, const float *__restrict__ wts,
-                               int64_t T, int n_used, int64_t M,
-                               const float *__restrict__ residual, float *__restrict__ out) {
-  const int64_t m = 4 * (blockIdx.x * (int64_t)blockDim.x + threadIdx.x);
-  if (m >= M) return;
-  for (int64_t t = blockIdx.y * (int64_t)blockDim.y + threadIdx.y; t < T;
-       t += (int64_t)gridDim.y * blockDim.y) {
-    const float *yt = y + t * n_used * M + m, *wt = wts + t * n_used;
-    const int64_t o = t * M + m;
-    if (m + 4 <= M) {
-      f32x4 s = {0, 0, 0, 0};
-      int j = 0;
-      for (; j + 8 <= n_used; j += 8) {
-        f32x4 v[8];
+__global__ void __launch_bounds__(ROW_BLOCK)
+moe_sum_kernel(const float *__restrict__ y, const float *__restrict__ wts, int64_t T, int n_used,
+               int64_t M, const float *__restrict__ residual, float *__restrict__ out) {
+  const int64_t m = 4 * (blockIdx.x * (int64_t)blockDim.x + threadIdx.x), t = row_of();
+  if (m >= M || t >= T) return;
+  const float *yt = y + t * n_used * M + m, *wt = wts + t * n_used;
+  const int64_t o = t * M + m;
+  if (m + 4 <= M) {
+    f32x4 s = {0, 0, 0, 0};
+    int j = 0;
+    for (; j + 8 <= n_used; j += 8) {
+      f32x4 v[8];
 #pragma unroll
-        for (int i = 0; i < 8; i++) v[i] = *(const f32x4_u *)(yt + (j + i) * M);
+      for (int i = 0; i < 8; i++) v[i] = *(const f32x4_u *)(yt + (j + i) * M);
 #pragma unroll
-        for (int i = 0; i < 8; i++) s += v[i] * wt[j + i];
-      }
-      for (; j < n_used; j++) s += *(const f32x4_u *)(yt + j * M) * wt[j];
-      if (residual) s += *(const f32x4_u *)(residual + o);
-      *(f32x4_u *)(out + o) = s;
-    } else {
-      for (int e = 0; m + e < M; e++) {
-        float s = 0.0f;
-        for (int j = 0; j < n_used; j++) s += yt[j * M + e] * wt[j];
-        out[o + e] = residual ? s + residual[o + e] : s;
-      }
+      for (int i = 0; i < 8; i++) s += v[i] * wt[j + i];
+    }
+    for (; j < n_used; j++) s += *(const f32x4_u *)(yt + j * M) * wt[j];
+    if (residual) s += *(const f32x4_u *)(residual + o);
+    *(f32x4_u *)(out + o) = s;
+  } else {
+    for (int e = 0; m + e < M; e++) {
+      float s = 0.0f;
+      for (int j = 0; j < n_used; j++) s += yt[j * M + e] * wt[j];
+      out[o + e] = residual ? s + residual[o + e] : s;
     }
   }
 }

@@ -31,26 +31,23 @@ int hip_check(hipError_t e, const char *what) {
 // from HBM); with a workgroup walking a row 256 values at a time that chain ran
 // 16 times at 4096 columns (15.4 us for 64 Q4_K rows; a decode pass of two layers
 // and the head 688 us so, 676 here).
-__global__ void get_rows_kernel(int type, const uint8_t *__restrict__ table, int64_t rb,
-                                int64_t n_cols, const int32_t *__restrict__ ids, int64_t n,
-                                float *__restrict__ out, float scale) {
-  const int64_t k0 = 4 * (blockIdx.x * (int64_t)blockDim.x + threadIdx.x);
-  if (k0 >= n_cols) return;
-  for (int64_t j = blockIdx.y * (int64_t)blockDim.y + threadIdx.y; j < n;
-       j += (int64_t)gridDim.y * blockDim.y) {
-    const uint8_t *row = table + (int64_t)ids[j] * rb;
-    float *o = out + j * n_cols + k0;
-    f32x4 v;
+__global__ void __launch_bounds__(ROW_BLOCK)
+get_rows_kernel(int type, const uint8_t *__restrict__ table, int64_t rb, int64_t n_cols,
+                const int32_t *__restrict__ ids, int64_t n, float *__restrict__ out, float scale) {
+  const int64_t k0 = 4 * (blockIdx.x * (int64_t)blockDim.x + threadIdx.x), j = row_of();
+  if (k0 >= n_cols || j >= n) return;
+  const uint8_t *row = table + (int64_t)ids[j] * rb;
+  float *o = out + j * n_cols + k0;
+  f32x4 v;
 #pragma unroll
-    for (int e = 0; e < 4; e++) {
-      v[e] = row_value(type, row, k0 + e < n_cols ? k0 + e : n_cols - 1);
-      if (scale != 0.0f) v[e] *= scale;
-    }
-    if (k0 + 4 <= n_cols) {
-      *(f32x4_u *)o = v;
-    } else {
-      for (int e = 0; k0 + e < n_cols; e++) o[e] = v[e];
-    }
+  for (int e = 0; e < 4; e++) {
+    v[e] = row_value(type, row, k0 + e < n_cols ? k0 + e : n_cols - 1);
+    if (scale != 0.0f) v[e] *= scale;
+  }
+  if (k0 + 4 <= n_cols) {
+    *(f32x4_u *)o = v;
+  } else {
+    for (int e = 0; k0 + e < n_cols; e++) o[e] = v[e];
   }
 }
 
@@ -337,75 +334,70 @@ __device__ __forceinline__ double glu_act(double g, int gelu) {
 // divided. Bound by its f64 arithmetic: 512 x 10240 gelu 39.5 us with one
 // value per thread, 64-bit divisions and an f64 tanh, 14.6 here.
 template <typename OutT>
-__global__ void swiglu_kernel(const float *__restrict__ gu, int64_t n, int64_t F,
-                              OutT *__restrict__ out, Pending pend, int gelu) {
-  const int64_t c = 4 * (blockIdx.x * (int64_t)blockDim.x + threadIdx.x);
-  if (c >= F) return;
+__global__ void __launch_bounds__(ROW_BLOCK)
+swiglu_kernel(const float *__restrict__ gu, int64_t n, int64_t F, OutT *__restrict__ out,
+              Pending pend, int gelu) {
+  const int64_t c = 4 * (blockIdx.x * (int64_t)blockDim.x + threadIdx.x), r = row_of();
+  if (c >= F || r >= n) return;
   const int w = F - c < 4 ? (int)(F - c) : 4;
-  for (int64_t r = blockIdx.y * (int64_t)blockDim.y + threadIdx.y; r < n;
-       r += (int64_t)gridDim.y * blockDim.y) {
-    float g[4] = {0, 0, 0, 0}, u[4] = {0, 0, 0, 0};
-    const float *gr = gu + r * 2 * F + c, *ur = gr + F;
-    if (pend.splits) {
-      for (int e = 0; e < w; e++) {
-        g[e] = pend.sum(r, c + e);
-        u[e] = pend.sum(r, F + c + e);
-      }
-    } else if (w == 4) {
-      const f32x4 a = *(const f32x4_u *)gr, b = *(const f32x4_u *)ur;
-#pragma unroll
-      for (int e = 0; e < 4; e++) {
-        g[e] = a[e];
-        u[e] = b[e];
-      }
-    } else {
-      for (int e = 0; e < w; e++) {
-        g[e] = gr[e];
-        u[e] = ur[e];
-      }
+  float g[4] = {0, 0, 0, 0}, u[4] = {0, 0, 0, 0};
+  const float *gr = gu + r * 2 * F + c, *ur = gr + F;
+  if (pend.splits) {
+    for (int e = 0; e < w; e++) {
+      g[e] = pend.sum(r, c + e);
+      u[e] = pend.sum(r, F + c + e);
     }
-    float v[4];
+  } else if (w == 4) {
+    const f32x4 a = *(const f32x4_u *)gr, b = *(const f32x4_u *)ur;
 #pragma unroll
     for (int e = 0; e < 4; e++) {
-      v[e] = (float)(glu_act(g[e], gelu) * (double)u[e]);
-      // An f16 output is f16 of this f32 value. Left free, the compiler folds
-      // the two conversions into one f64 -> f16 rounding, which differs at
-      // f16 ties (rounding an arbitrary f64 value twice is not innocuous).
-      asm volatile("" : "+v"(v[e]));
+      g[e] = a[e];
+      u[e] = b[e];
     }
-    OutT *o = out + r * F + c;
-    if (w == 4) {
-      typedef OutT o4 __attribute__((ext_vector_type(4), aligned(sizeof(OutT))));
-      *(o4 *)o = o4{(OutT)v[0], (OutT)v[1], (OutT)v[2], (OutT)v[3]};
-    } else {
-      for (int e = 0; e < w; e++) o[e] = (OutT)v[e];
+  } else {
+    for (int e = 0; e < w; e++) {
+      g[e] = gr[e];
+      u[e] = ur[e];
     }
+  }
+  float v[4];
+#pragma unroll
+  for (int e = 0; e < 4; e++) {
+    v[e] = (float)(glu_act(g[e], gelu) * (double)u[e]);
+    // An f16 output is f16 of this f32 value. Left free, the compiler folds
+    // the two conversions into one f64 -> f16 rounding, which differs at
+    // f16 ties (rounding an arbitrary f64 value twice is not innocuous).
+    asm volatile("" : "+v"(v[e]));
+  }
+  OutT *o = out + r * F + c;
+  if (w == 4) {
+    typedef OutT o4 __attribute__((ext_vector_type(4), aligned(sizeof(OutT))));
+    *(o4 *)o = o4{(OutT)v[0], (OutT)v[1], (OutT)v[2], (OutT)v[3]};
+  } else {
+    for (int e = 0; e < w; e++) o[e] = (OutT)v[e];
   }
 }
 
 // The same values into X planes (F % 256 == 0); a thread per 8 values.
-__global__ void swiglu_split_kernel(const float *__restrict__ gu, int64_t n, int64_t F,
-                                    f16 *__restrict__ planes, int64_t npad, Pending pend,
-                                    int gelu, int xf) {
-  const int64_t c0 = 8 * (blockIdx.x * (int64_t)blockDim.x + threadIdx.x);
-  if (c0 >= F) return;  // whole blocks of lanes leave together
-  for (int64_t r = blockIdx.y * (int64_t)blockDim.y + threadIdx.y; r < n;
-       r += (int64_t)gridDim.y * blockDim.y) {
-    float g8[8], u8[8], v[8];
-    if (pend.splits) {
-      pend.sum8(r, c0, g8);
-      pend.sum8(r, F + c0, u8);
-    } else {
+__global__ void __launch_bounds__(ROW_BLOCK)
+swiglu_split_kernel(const float *__restrict__ gu, int64_t n, int64_t F, f16 *__restrict__ planes,
+                    int64_t npad, Pending pend, int gelu, int xf) {
+  const int64_t c0 = 8 * (blockIdx.x * (int64_t)blockDim.x + threadIdx.x), r = row_of();
+  if (c0 >= F || r >= n) return;  // whole blocks of lanes leave together
+  float g8[8], u8[8], v[8];
+  if (pend.splits) {
+    pend.sum8(r, c0, g8);
+    pend.sum8(r, F + c0, u8);
+  } else {
 #pragma unroll
-      for (int e = 0; e < 8; e++) {
-        g8[e] = gu[r * 2 * F + c0 + e];
-        u8[e] = gu[r * 2 * F + F + c0 + e];
-      }
+    for (int e = 0; e < 8; e++) {
+      g8[e] = gu[r * 2 * F + c0 + e];
+      u8[e] = gu[r * 2 * F + F + c0 + e];
     }
-#pragma unroll
-    for (int e = 0; e < 8; e++) v[e] = (float)(glu_act(g8[e], gelu) * (double)u8[e]);
-    act_store8(xf, planes, npad, F, r, c0, v);
   }
+#pragma unroll
+  for (int e = 0; e < 8; e++) v[e] = (float)(glu_act(g8[e], gelu) * (double)u8[e]);
+  act_store8(xf, planes, npad, F, r, c0, v);
 }
 
 // ---- logit softcap: cap * tanh(x * (1 / cap)) (transformer.lua:2097-2099) ----
