@@ -1623,7 +1623,7 @@ int split_x(const void *x, int xtype, int64_t N, int64_t K, f16 *xs, hipStream_t
     return LGMLH_EINVAL;
   }
   if (N * K == 0) return LGMLH_OK;
-  const RowGrid g(K / 8, N);
+  const RowGrid g(K / 8, N, 32);  // 32 lanes hold a 256-value block
   hipLaunchKernelGGL(xsplit_kernel, g.grid, g.block, 0, st, x, xtype, N, K, xs, split_npad(N), xf);
   return hip_check(hipGetLastError(), "split");
 }

@@ -524,7 +524,7 @@ int swiglu_dev(const float *gu, int64_t n, int64_t F, float *out, f16 *planes, h
       set_error("swiglu: split output needs F %% 256 == 0 (F = %lld)", (long long)F);
       return LGMLH_EINVAL;
     }
-    const RowGrid g(F / 8, n);
+    const RowGrid g(F / 8, n, 32);  // 32 lanes hold a 256-value block
     hipLaunchKernelGGL(swiglu_split_kernel, g.grid, g.block, 0, st, gu, n, F, planes,
                        split_npad(n), pend, gelu, xf);
   }

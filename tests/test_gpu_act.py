@@ -40,9 +40,10 @@ def act_rows(K, n, seed):
 
 
 @pytest.mark.parametrize("ty", [core.Q4_K, core.Q8_0])
-def test_quantize_act_bit_exact(L, ty):
+@pytest.mark.parametrize("K,n", [(1024, 37), (256, 21), (512, 5), (768, 9), (2304, 6), (3840, 4)])
+def test_quantize_act_bit_exact(L, ty, K, n):
+    """Rows of whole and of part-filled workgroups, one to eight to each."""
     from lgml_amd import hip
-    K, n = 1024, 37
     x = act_rows(K, n, 1)
     qd = torch.empty((n, K), dtype=torch.int8, device="cuda")
     if ty == core.Q8_0:

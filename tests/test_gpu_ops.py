@@ -276,7 +276,7 @@ def test_get_rows(L, ty):
 
 
 @pytest.mark.parametrize("ty,cols,n", [
-    (core.F32, 1, 5), (core.F32, 1027, 3), (core.F16, 259, 9), (core.F16, 2, 300),
+    (core.F32, 1, 5), (core.F32, 9, 65535 * 4 + 7), (core.F32, 1027, 3), (core.F16, 259, 9), (core.F16, 2, 300),
     (core.Q8_0, 32, 1), (core.Q8_0, 1056, 6), (core.Q4_K, 256, 2), (core.Q6_K, 4352, 3)])
 def test_get_rows_ragged_columns(L, ty, cols, n):
     """Columns that end inside a thread's four and inside a workgroup."""
