@@ -1474,9 +1474,15 @@ static int launch_q(const void *w, int64_t M, int64_t K, const f16 *xs, int64_t 
   // 2.29 ms, the pass 0.4 ms shorter than with pairs from 512 tiles).
   // A product of two splits whose sums nobody else adds (the plain entry
   // points) runs them in one workgroup from 1024 workgroups up: no partial
-  // sums and no reduction launch (Q8_0 20480 x 2560 at 512 rows 165 -> 152 us,
-  // Q6_K 141 -> 123; with more splits the reduction stays and the pairs only
-  // make fewer rounds: Q4_K 4096 x 14336 at 575 rows 120 -> 128).
+  // sums and no reduction launch. Whole products in ggml's arithmetic in us, with
+  // two workgroups and a reduction (up to 4 us longer than it is now) / with one:
+  // at 1024 workgroups 16384 x 4096, 512 rows Q4_K 119 / 105, Q6_K 163 / 150,
+  // Q8_0 178 / 150; at 1088 8192 x 1024, 1088 rows 63 / 51, 73 / 63, 90 / 65; at
+  // 1120 14336 x 1024, 600 rows 62 / 51, 72 / 63, 89 / 65; at 1280 20480 x 2560, 512
+  // rows 107 / 91, 141 / 124, 157 / 126 (Q8_0 with its 8-wave workgroups before);
+  // at 1904 14336 x 4096, 1088 rows 212 / 194, 296 / 277, 341 / 284. (With more
+  // splits the reduction stays and the pairs only make fewer rounds: Q4_K
+  // 4096 x 14336 at 575 rows 120 -> 128.)
   const bool can_fold = splits > 1 && nct == 4 && (TYPE != LGMLH_Q8_0 || Q8);
   const int fold = can_fold && ((TYPE != LGMLH_Q8_0 && tiles * splits >= 8192) ||
                                 (!defer && splits == SPLIT_PAIR && tiles >= 1024))
