@@ -469,7 +469,8 @@ qgemm_kernel(const uint8_t *__restrict__ w, int64_t M, int64_t K, const f16 *__r
 #pragma unroll
     for (int j = 0; j < XJ; j++) {
       const int slot0 = (wave * XJ + j) * 64;
-      if (NCT == 4 && GATHER && slot0 >= live * 16 * 32) continue;  // a column tile without picks
+      // a column tile without picks
+      if (NCT == 4 && GATHER && live < NCT && slot0 >= live * 16 * 32) continue;
       // a wave-uniform base plus a 32-bit lane offset (no 64-bit adds per lane)
       const uint8_t *bh = (const uint8_t *)(xhi + kstep * QK_K);
       const uint8_t *bl = (const uint8_t *)(xlo + kstep * QK_K);
@@ -822,7 +823,15 @@ qgemm_kernel(const uint8_t *__restrict__ w, int64_t M, int64_t K, const f16 *__r
   else
     emit(out, ld_out, false, nz == 1 && residual);
   };
-  if constexpr (GATHER && NCT == 4) {
+  // (Q8_0 with split X has no registers to spare: all four lengths spill 4 and
+  // take 95 us where two take 88, 512 x 8 picks over 8 experts of 1536 x 2048;
+  // twelve spilled with the column test in the full length, 113.)
+  if constexpr (GATHER && NCT == 4 && TYPE == LGMLH_Q8_0 && !Q8) {
+    if (count > 32)
+      run(std::integral_constant<int, 4>{});
+    else
+      run(std::integral_constant<int, 2>{});
+  } else if constexpr (GATHER && NCT == 4) {
     if (count > 48)
       run(std::integral_constant<int, 4>{});
     else if (count > 32)

@@ -35,3 +35,13 @@ def test_row_kernels_keep_their_values_in_registers(name):
     assert got
     for n, k in got.items():
         assert k[".private_segment_fixed_size"] == 0 and k.get(".vgpr_spill_count", 0) == 0, n
+
+
+def test_grouped_wide_tiles_spill_next_to_nothing():
+    """The 64-column grouped products run at 256 registers: Q8_0 with split X
+    spills three, the others none (twelve made it a quarter slower)."""
+    got = {n: k for n, k in kernels().items() if "qgemm_kernelILi" in n and "ELi4ELb1E" in n}
+    assert len(got) == 6
+    for n, k in got.items():
+        q80_exact = "ILi8ELi4ELb1ELb0E" in n
+        assert k[".private_segment_fixed_size"] <= (16 if q80_exact else 0), n
