@@ -11,9 +11,9 @@
 // f32 (each lane owns one row; reductions over 4 lanes with shuffles), and
 // O^T += V^T P^T (V columns straight from the transposed [D][cell] tile, P
 // from the lane's own S^T values: s_cell). K and V are exact f16; Q and P
-// enter the MFMAs as f16 hi + lo pairs, P held ATTN_P times as large (l and O
-// with it: the factor cancels), so that a pair carries 22 bits of every P down
-// to 2^-17 of the row's largest, and below is at most 2^-40 of that off.
+// enter the MFMAs as f16 hi + lo pairs, P ATTN_P times as large (O with it, and
+// l in the end: the factor cancels), so that a pair carries 22 bits of every P
+// down to 2^-17 of the row's largest, and below is at most 2^-40 of that off.
 // (Unscaled, P below 2^-25 was 0 in O but counted in l: one cell 16 above 2000
 // others made 4% to 20% of the result wrong. 64 decoding sequences of 32 / 8
 // heads of 128 take 106 us either way, a 512-token chunk beside 32 sequences
@@ -98,7 +98,7 @@ __device__ __forceinline__ void softmax_block(f32x4 (&st)[4], float scale_log2, 
   for (int ct = 0; ct < 4; ct++)
 #pragma unroll
     for (int i = 0; i < 4; i++) {
-      st[ct][i] = __builtin_amdgcn_exp2f(st[ct][i] - m_use) * ATTN_P;  // exp2(-inf) = 0
+      st[ct][i] = __builtin_amdgcn_exp2f(st[ct][i] - m_use);  // exp2(-inf) = 0
       rs += st[ct][i];
     }
   rs += __shfl_xor(rs, 16);
@@ -117,7 +117,8 @@ __device__ __forceinline__ void softmax_block(f32x4 (&st)[4], float scale_log2, 
   for (int j = 0; j < 2; j++)
 #pragma unroll
     for (int e = 0; e < 8; e += 2) {
-      const f32x2 p = {st[2 * j + (e >> 2)][e & 3], st[2 * j + (e >> 2)][(e & 3) + 1]};
+      const f32x2 p = {st[2 * j + (e >> 2)][e & 3] * ATTN_P,
+                       st[2 * j + (e >> 2)][(e & 3) + 1] * ATTN_P};
       const f16x2 hi = __builtin_convertvector(p, f16x2);
       const f32x2 r = {fmaf((float)hi[0], -1.0f, p[0]), fmaf((float)hi[1], -1.0f, p[1])};
       const f16x2 lo = __builtin_convertvector(r, f16x2);
@@ -407,10 +408,11 @@ paged_attn_kernel(const float *__restrict__ q, int H, int Hkv, float scale_log2,
   // (straight-line code keeps the load counter waits exact, so the O
   // products do not wait for the next K). Heads of up to 128 run the last
   // block without NEXT, so no tile is loaded twice; heads of 256 (whose
-  // registers are full) load the last block's tiles again, from L2
-  // (whose schedule is held in program order: left free, tiles in flight
-  // spilled, and a spill waits for them: 214 -> 260 us at 32 sequences of
-  // U[1024, 16384]).
+  // registers are full) load the last block's tiles again, from L2. Their O
+  // products stay behind the softmax: with the schedule free, tiles in flight
+  // spilled, and a spill waits for them (214 -> 260 us at 32 sequences of
+  // U[1024, 16384]); held in program order after S and after O too, a chain of
+  // few blocks is longer (one sequence of 2386 cells 43.7 us, 38.6 so).
   constexpr bool PEEL = D <= 128;
   auto block = [&](int blk, auto next) __attribute__((always_inline)) {
     constexpr bool NEXT = decltype(next)::value;
@@ -427,7 +429,6 @@ paged_attn_kernel(const float *__restrict__ q, int H, int Hkv, float scale_log2,
       }
       st[ct] = acc;
     }
-    if constexpr (!PEEL) __builtin_amdgcn_sched_barrier(0);
     if constexpr (NEXT) load_k(ktile(nxt));
 
     // A block that ends at or before the group's first position (and, with a
@@ -447,14 +448,13 @@ paged_attn_kernel(const float *__restrict__ q, int H, int Hkv, float scale_log2,
         o[dt] = mfma16(vf[dt][kc], pfh[kc], o[dt]);
         o[dt] = mfma16(vf[dt][kc], pfl[kc], o[dt]);
       }
-    if constexpr (!PEEL) __builtin_amdgcn_sched_barrier(0);
     if constexpr (NEXT) load_v(vtile(nxt));
   };
   for (int blk = blo; blk + (PEEL ? 1 : 0) < bhi; blk++) block(blk, std::true_type{});
   if constexpr (PEEL)
     if (blo < bhi) block(bhi - 1, std::false_type{});
 
-  finish_item<D>(o, m, l, mg, rvalid, tok0, rtok, rhead, ntok, G, row, quad, item, kvh, Hkv, H,
+  finish_item<D>(o, m, l * ATTN_P, mg, rvalid, tok0, rtok, rhead, ntok, G, row, quad, item, kvh, Hkv, H,
                  out, planes, npad, xf, part);
 }
 
@@ -626,7 +626,7 @@ paged_attn_shared_kernel(const float *__restrict__ q, int H, int Hkv, float scal
     __syncthreads();                // ... and everyone's; buffer buf is free again
   }
   if (!active) return;
-  finish_item<D>(o, m, l, mg, rvalid, tok0, rtok, rhead, ntok, G, row, quad, item, kvh, Hkv, H,
+  finish_item<D>(o, m, l * ATTN_P, mg, rvalid, tok0, rtok, rhead, ntok, G, row, quad, item, kvh, Hkv, H,
                  out, planes, npad, xf, part);
 }
 
