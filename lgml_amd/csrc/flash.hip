@@ -15,8 +15,8 @@
 //
 // K and V are exact f16; Q and P enter the MFMAs as f16 hi + lo pairs, with
 // the largest of a row near f16's (Q by a power of two per row, so any f32
-// row fits; P is held FA_P times as large, l and O with it, so that the
-// factor cancels) and the low parts FA_LO times as large again, with products
+// row fits; P FA_P times as large, O with it, and l in the end: the factor
+// cancels) and the low parts FA_LO times as large again, with products
 // of their own: a pair carries 22 bits of every value down to 2^-28 of the
 // row's largest, and what is lost below is at most 2^-51 of that. (With the
 // largest at 1 and one sum for both, q values below 2^-14 of it lost bits: rows
@@ -399,8 +399,7 @@ __global__ void __launch_bounds__(RW *KW * 64, 1) flash_attn_kernel(FlashArgs A)
     for (int ct = 0; ct < CT; ct++)
 #pragma unroll
       for (int i = 0; i < 4; i++) {
-        // exp2(-inf) = 0
-        st[ct][i] = __builtin_amdgcn_exp2f((st[ct][i] - m_use) * FA_LOG2E) * FA_P;
+        st[ct][i] = __builtin_amdgcn_exp2f((st[ct][i] - m_use) * FA_LOG2E);  // exp2(-inf) = 0
         rs += st[ct][i];
       }
     rs += __shfl_xor(rs, 16);
@@ -418,7 +417,8 @@ __global__ void __launch_bounds__(RW *KW * 64, 1) flash_attn_kernel(FlashArgs A)
     for (int j = 0; j < CJ; j++)
 #pragma unroll
       for (int e = 0; e < 8; e += 2) {
-        const f32x2 p = {st[2 * j + (e >> 2)][e & 3], st[2 * j + (e >> 2)][(e & 3) + 1]};
+        const f32x2 p = {st[2 * j + (e >> 2)][e & 3] * FA_P,
+                         st[2 * j + (e >> 2)][(e & 3) + 1] * FA_P};
         const f16x2 hi = __builtin_convertvector(p, f16x2);
         const f32x2 r = {(p[0] - (float)hi[0]) * FA_LO, (p[1] - (float)hi[1]) * FA_LO};
         const f16x2 lo = __builtin_convertvector(r, f16x2);
@@ -476,7 +476,7 @@ __global__ void __launch_bounds__(RW *KW * 64, 1) flash_attn_kernel(FlashArgs A)
 #pragma unroll
           for (int i = 0; i < 4; i++)
             if (c == ct * 16 + (c & 12) + i) p = st[ct][i];
-        p = __shfl(p, ((c & 12) >> 2) * 16 + r16);
+        p = __shfl(p, ((c & 12) >> 2) * 16 + r16) * FA_P;
         const uint16_t *vs = vb + (int64_t)min(tile * BC + c, A.n_kv - 1) * A.v_rs;
 #pragma unroll
         for (int dt = 0; dt < DT; dt++)
@@ -582,7 +582,7 @@ __global__ void __launch_bounds__(RW *KW * 64, 1) flash_attn_kernel(FlashArgs A)
   }
   if (rvalid && l == l) {
     // a row with every cell masked gives zeros
-    const float inv = l == 0.0f ? 0.0f : 1.0f / l;
+    const float inv = l == 0.0f ? 0.0f : 1.0f / (l * FA_P);
     float *orow = A.out + ((int64_t)t * A.H + h) * D;
 #pragma unroll
     for (int dt = 0; dt < DT; dt++) {
