@@ -101,9 +101,17 @@ __device__ void exact_row(const FlashArgs &A, int kvh, uint32_t rr) {
     const float mv = j >= A.n_kv ? -INFINITY : mr ? h2f(mr[j]) : 0.0f;
     float s = -INFINITY;
     if (mv != -INFINITY) {
+      const uint16_t *kr = kb + (int64_t)j * A.k_rs;
       float a = 0.0f;
-#pragma unroll 1
-      for (int d = 0; d < A.D; d++) a = fmaf(qr[d], h2f(kb[(int64_t)j * A.k_rs + d]), a);
+#pragma unroll 4
+      for (int d = 0; d < A.D; d += 8) {
+        const u32x4 w = *(const u32x4 *)(kr + d);
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+          a = fmaf(qr[d + 2 * e], h2f((uint16_t)(w[e] & 0xffffu)), a);
+          a = fmaf(qr[d + 2 * e + 1], h2f((uint16_t)(w[e] >> 16)), a);
+        }
+      }
       a *= sc;
       if (A.softcap > 0.0f) a = A.softcap * tanhf(a);
       s = a + slope * mv;
@@ -119,13 +127,21 @@ __device__ void exact_row(const FlashArgs &A, int kvh, uint32_t rr) {
     for (int i = 0; i < FA_MAX_D / 64; i++) o[i] *= corr;
     const int nj = min(A.n_kv - j0, 64);
 #pragma unroll 1
-    for (int jj = 0; jj < nj; jj++) {
-      const float pj = __shfl(p, jj);
-      if (pj == 0.0f) continue;  // wave-uniform
-      const uint16_t *vr = vb + (int64_t)(j0 + jj) * A.v_rs;
+    for (int j1 = 0; j1 < nj; j1 += 4) {  // four cells' values in flight
+      uint16_t x[4][FA_MAX_D / 64];
 #pragma unroll
-      for (int i = 0; i < FA_MAX_D / 64; i++)
-        if (lane + 64 * i < A.D) o[i] = fmaf(pj, h2f(vr[lane + 64 * i]), o[i]);
+      for (int c = 0; c < 4; c++) {
+        const uint16_t *vr = vb + (int64_t)(j0 + min(j1 + c, nj - 1)) * A.v_rs;
+#pragma unroll
+        for (int i = 0; i < FA_MAX_D / 64; i++) x[c][i] = lane + 64 * i < A.D ? vr[lane + 64 * i] : 0;
+      }
+#pragma unroll
+      for (int c = 0; c < 4; c++) {
+        const float pj = __shfl(p, j1 + c);
+        if (pj == 0.0f || j1 + c >= nj) continue;  // wave-uniform
+#pragma unroll
+        for (int i = 0; i < FA_MAX_D / 64; i++) o[i] = fmaf(pj, h2f(x[c][i]), o[i]);
+      }
     }
     m = mn;
   }
@@ -134,6 +150,11 @@ __device__ void exact_row(const FlashArgs &A, int kvh, uint32_t rr) {
 #pragma unroll
   for (int i = 0; i < FA_MAX_D / 64; i++)
     if (lane + 64 * i < A.D) orow[lane + 64 * i] = o[i] * inv;
+}
+
+// Calls of few cells: a wave per row.
+__global__ void __launch_bounds__(64) flash_row_kernel(FlashArgs A) {
+  exact_row(A, blockIdx.y, blockIdx.x);
 }
 
 // DP: the head size padded to the MFMA step (zeros past D); BC: cells per
@@ -614,9 +635,20 @@ static void launch_flash(const FlashArgs &A, int n_head_kv, hipStream_t st) {
 // K straight from memory. (32 / 8 heads of 128, 2048 cells: 200 rows, 104
 // workgroups of 64 rows, 64.6 us; 100 rows as 16-row workgroups 40.7; one
 // row 36.4, 670 in the wave-per-row kernel before.) A single 32-cell tile
-// needs one wave: nothing to merge.
+// needs one wave: nothing to merge. And a wave per row where the cells are fewer than
+// a tile's setup takes: up to 4 cells of 2048 rows in all (in us, a tile / a
+// wave per row: one row of 32 heads of 64 over 4 cells 5.3 / 4.0, of 256 10.0 /
+// 6.4, 64 rows of 8 heads of 16 4.8 / 4.0; 512 rows of 8 heads of 16 4.9 / 5.4),
+// from heads of 64 up to 8 cells of 512 rows (one row of 32 heads of 64 over 8
+// 5.3 / 4.8, 12 5.3 / 5.7; 64 rows of 32 heads over 8 5.6 / 5.8).
 template <int DP>
 static void flash_for(const FlashArgs &A, int n_head_kv, hipStream_t st) {
+  const int64_t rows = (int64_t)A.T * A.G * n_head_kv;
+  if (A.n_kv <= 4 ? rows <= 2048 : A.n_kv <= 8 && DP >= 64 && rows <= 512) {
+    hipLaunchKernelGGL(flash_row_kernel, dim3((unsigned)(A.T * A.G), (unsigned)n_head_kv), dim3(64),
+                       0, st, A);
+    return;
+  }
   const int64_t tiles = ((int64_t)A.T * A.G + 63) / 64 * n_head_kv;
   constexpr int WIDE = DP <= 128 ? 2 : 1, SPLIT = DP <= 128 ? 8 : 4;
   if (tiles >= 96)

@@ -300,6 +300,32 @@ def test_flash_attn_seen_infinities_in_q_and_k(L, T, D, softcap):
     assert 2 * T < n_nan < 4 * T  # heads 12 and 13, which see the NaN, and single rows
 
 
+# The switch between a wave per row and tiles: up to 4 cells of 2048 rows in all,
+# from heads of 64 up to 8 cells of 512 rows.
+@pytest.mark.parametrize("H,Hkv,T,D,n_kv", [
+    (4, 2, 512, 16, 1), (4, 2, 513, 16, 2), (4, 1, 512, 40, 4), (4, 2, 3, 40, 5),
+    (8, 2, 64, 64, 5), (8, 2, 65, 64, 8), (2, 1, 256, 128, 8), (2, 1, 5, 128, 9),
+    (8, 8, 1, 256, 3), (6, 2, 11, 200, 7)])
+def test_flash_attn_few_cells(L, H, Hkv, T, D, n_kv):
+    rng = np.random.default_rng(66)
+    q = rng.standard_normal((H, T, D)).astype(np.float32)
+    k = core.f32_to_f16_bits(rng.standard_normal((Hkv, n_kv, D)).astype(np.float32))
+    v = rng.standard_normal((Hkv, n_kv, D)).astype(np.float32)
+    m = np.where(rng.random((2, T, n_kv)) < 0.5, rng.random((2, T, n_kv)), -np.inf)
+    m[:, :, 0] = 0.25
+    m[1, T - 1] = -np.inf  # a row that sees nothing
+    mask = core.f32_to_f16_bits(m.astype(np.float32))
+    want = core.flash_attn(q, k, core.f32_to_f16_bits(v), Hkv, mask, D ** -0.5, 2.0, 15.0)
+    if n_kv > 1:  # what no row sees may hold anything
+        m[:, :, n_kv - 1] = -np.inf
+        mask = core.f32_to_f16_bits(m.astype(np.float32))
+        want = core.flash_attn(q, k, core.f32_to_f16_bits(v), Hkv, mask, D ** -0.5, 2.0, 15.0)
+        v[:, n_kv - 1] = np.nan
+    got = gpu_flash(L, q, k, core.f32_to_f16_bits(v), Hkv, n_kv, (D, n_kv * D), (D, n_kv * D), mask,
+                    D ** -0.5, 2.0, 15.0)
+    assert rel_err(got.reshape(T * H, D) + 1e-30, want.reshape(T * H, D) + 1e-30) < 1e-5
+
+
 def test_flash_attn_addresses_of_elements(L):
     """q, v, the mask and out start at any element (k is 16-byte aligned)."""
     from lgml_amd import hip
