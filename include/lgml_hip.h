@@ -259,7 +259,10 @@ int lgmlh_paged_attention(const float *q, int n_head, int n_head_kv, int head_di
  * in elements, K 16-byte aligned with strides multiples of 8); mask
  * (mask_heads, mask_rows >= T, n_kv) contiguous f16 or NULL; out (T, H, D)
  * f32 (heads and tokens swapped, as the reference returns). Head h reads
- * kv head h / (H / Hkv). D a multiple of 8 up to 256. */
+ * kv head h / (H / Hkv). D a multiple of 8 up to 256. Unlike the paged entry
+ * it is not batch invariant: the number of rows of a call picks its kernel,
+ * so a row's last bits may differ between calls of different T (within f32
+ * rounding); calls of the same shape repeat them. */
 int lgmlh_flash_attn(const float *q, int n_head, int n_tokens, int head_dim, const uint16_t *k,
     const uint16_t *v, int n_head_kv, int n_kv, int64_t k_row_stride, int64_t k_head_stride,
     int64_t v_row_stride, int64_t v_head_stride, const uint16_t *mask, int mask_heads,

@@ -326,6 +326,23 @@ def test_flash_attn_few_cells(L, H, Hkv, T, D, n_kv):
     assert rel_err(got.reshape(T * H, D) + 1e-30, want.reshape(T * H, D) + 1e-30) < 1e-5
 
 
+@pytest.mark.parametrize("H,Hkv,T,D,n_kv,parts", [
+    (32, 8, 200, 64, 300, (1, 176, 177)),  # 4 row tiles of 16 a workgroup from 177 rows up
+    (8, 8, 300, 128, 6, (64, 65, 300))])   # a wave per row up to 64 rows
+def test_flash_attn_rows_in_calls_of_other_sizes(L, H, Hkv, T, D, n_kv, parts):
+    """A row's last bits depend on the kernel that the number of rows picks:
+    within the f32 bound of the tile edges it is the same in any call."""
+    rng = np.random.default_rng(67)
+    q = rng.standard_normal((H, T, D)).astype(np.float32)
+    k = core.f32_to_f16_bits(rng.standard_normal((Hkv, n_kv, D)).astype(np.float32))
+    v = core.f32_to_f16_bits(rng.standard_normal((Hkv, n_kv, D)).astype(np.float32))
+    whole = gpu_flash(L, q, k, v, Hkv, n_kv, (D, n_kv * D), (D, n_kv * D), None, D ** -0.5)
+    for n in parts:
+        some = gpu_flash(L, np.ascontiguousarray(q[:, :n]), k, v, Hkv, n_kv, (D, n_kv * D),
+                         (D, n_kv * D), None, D ** -0.5)
+        assert rel_err(some.reshape(n * H, D), whole[:n].reshape(n * H, D)) < 1e-5, n
+
+
 def test_flash_attn_addresses_of_elements(L):
     """q, v, the mask and out start at any element (k is 16-byte aligned)."""
     from lgml_amd import hip
