@@ -633,13 +633,13 @@ static void launch_flash(const FlashArgs &A, int n_head_kv, hipStream_t st) {
 // fill LDS). Below, most CUs would stay idle: one row tile per workgroup,
 // its cells over 8 waves (4 past 128, whose registers take a SIMD each),
 // K straight from memory. (32 / 8 heads of 128, 2048 cells: 200 rows, 104
-// workgroups of 64 rows, 64.6 us; 100 rows as 16-row workgroups 40.7; one
-// row 36.4, 670 in the wave-per-row kernel before.) A single 32-cell tile
+// workgroups of 64 rows, 70 us; 100 rows as 16-row workgroups 40.6; one row
+// 36.9, 670 in the wave-per-row kernel before.) A single 32-cell tile
 // needs one wave: nothing to merge. And a wave per row where the cells are fewer than
 // a tile's setup takes: up to 4 cells of 2048 rows in all (in us, a tile / a
 // wave per row: one row of 32 heads of 64 over 4 cells 5.3 / 4.0, of 256 10.0 /
 // 6.4, 64 rows of 8 heads of 16 4.8 / 4.0; 512 rows of 8 heads of 16 4.9 / 5.4),
-// from heads of 64 up to 8 cells of 512 rows (one row of 32 heads of 64 over 8
+// for heads past 32 up to 8 cells of 512 rows (one row of 32 heads of 64 over 8
 // 5.3 / 4.8, 12 5.3 / 5.7; 64 rows of 32 heads over 8 5.6 / 5.8).
 template <int DP>
 static void flash_for(const FlashArgs &A, int n_head_kv, hipStream_t st) {

@@ -29,8 +29,8 @@ int hip_check(hipError_t e, const char *what) {
 // transformer.lua:2304-2306). Four values a thread, rows in blockIdx.y and
 // threadIdx.y: a launch is its chain of loads (the id, then the row's bytes
 // from HBM); with a workgroup walking a row 256 values at a time that chain ran
-// 16 times at 4096 columns (15.4 us for 64 Q4_K rows; a decode pass of two layers
-// and the head 688 us so, 676 here).
+// 16 times at 4096 columns (14.1 us for 64 Q4_K rows, 5.2 here; 512 rows 18.4
+// and 9.3).
 __global__ void __launch_bounds__(ROW_BLOCK)
 get_rows_kernel(int type, const uint8_t *__restrict__ table, int64_t rb, int64_t n_cols,
                 const int32_t *__restrict__ ids, int64_t n, float *__restrict__ out, float scale) {
@@ -332,7 +332,7 @@ __device__ __forceinline__ double glu_act(double g, int gelu) {
 // A thread's 4 consecutive values of a row; threads run along the row
 // (blockIdx.x), rows in blockIdx.y and threadIdx.y, so that no index is
 // divided. Bound by its f64 arithmetic: 512 x 10240 gelu 39.5 us with one
-// value per thread, 64-bit divisions and an f64 tanh, 14.6 here.
+// value per thread, 64-bit divisions and an f64 tanh, 13.2 here.
 template <typename OutT>
 __global__ void __launch_bounds__(ROW_BLOCK)
 swiglu_kernel(const float *__restrict__ gu, int64_t n, int64_t F, OutT *__restrict__ out,

@@ -301,7 +301,7 @@ def test_flash_attn_seen_infinities_in_q_and_k(L, T, D, softcap):
 
 
 # The switch between a wave per row and tiles: up to 4 cells of 2048 rows in all,
-# from heads of 64 up to 8 cells of 512 rows.
+# for heads past 32 up to 8 cells of 512 rows.
 @pytest.mark.parametrize("H,Hkv,T,D,n_kv", [
     (4, 2, 512, 16, 1), (4, 2, 513, 16, 2), (4, 1, 512, 40, 4), (4, 2, 3, 40, 5),
     (8, 2, 64, 64, 5), (8, 2, 65, 64, 8), (2, 1, 256, 128, 8), (2, 1, 5, 128, 9),
