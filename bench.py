@@ -1,7 +1,7 @@
 #!/usr/bin/env python3
 """Decode throughput of lgml's ragged continuous-batching path on one MI355X.
 
-Default workload (BASELINE.json configs[1], "C2"): a Llama-3-8B-shaped model
+Default workload ("C2"): a Llama-3-8B-shaped model
 (32 layers, d 4096, 32 / 8 heads, head 128, FFN 14336, vocab 128256) with
 N(0, 0.02) weights quantized Q4_K_M (output and attn_v / ffn_down of the
 more_bits layers Q6_K), f16 KV in 64-cell blocks; 64 slots with prompt
@@ -16,23 +16,23 @@ attention reads cost the same whatever the values); joining prompts run
 the real prefill. One step = one pass of the engine (E:flush): the next
 token of every decoding slot plus the prompt chunks of joining slots.
 
---workload c3 (BASELINE.json configs[2]): the same 8B model with prefix
+--workload c3: the same 8B model with prefix
 caching. A 2048-token system prefix is prefilled once and its 32 blocks
 are published; 64 requests of prefix + a unique suffix U[16, 512] attach
 those blocks (refcounts up to 64) and run only their suffixes; joins do
 the same, their suffix prefilled in 512-token chunks mixed into the
 decode pass (a pass carries the decode tokens and at most 512 prompt
 tokens). Attention bytes are reported both logical (every sequence's own
-context, the §8(d) figure the roofline uses) and unique (the shared
+context, the figure the roofline uses) and unique (the shared
 prefix once).
 
---workload c5 (BASELINE.json configs[4]): the same loop on a 30B-A3B-shaped
+--workload c5: the same loop on a 30B-A3B-shaped
 qwen3moe (48 layers, d 2048, 32 / 4 heads, head 128, 128 experts of width
 768, top-8 softmax routing, router logits N(0, 1), Q4_K), prompts
 U[256, 8192]: tokens are grouped by expert for the grouped Q4_K expert
 products.
 
---workload c4 (BASELINE.json configs[3]): a Gemma-4-style model (26 layers,
+--workload c4: a Gemma-4-style model (26 layers,
 d 2560, 8 / 4 heads of 256, 5 sliding-window layers with a 1024-token ring
 per slot to 1 global layer, GeGLU FFN 10240, vocab 262144 tied, Q8_0), 32
 slots with contexts U[1024, 16384] decoding (no joins: every budget

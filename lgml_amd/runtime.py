@@ -87,7 +87,7 @@ def repack_experts(gate, up, n_expert, K):
 
 def router_sd(hp):
     """Router weights N(0, 1 / sqrt(n_embd)): logits of a unit-rms h are then
-    N(0, 1) (BASELINE.json's MoE config)."""
+    N(0, 1)."""
     return 1.0 / float(np.sqrt(hp["n_embd"]))
 
 

@@ -1,5 +1,5 @@
 """Model shapes, weight-type policy and synthetic workloads of the benchmark
-configurations (BASELINE.json configs; seeds recorded with each result).
+configurations (seeds recorded with each result).
 
 Integers (lengths, ids, budgets) come from the reference's test LCG
 (test/tiny.lua:16-22); weights from lgmlh_gen_normal (tensor:fill

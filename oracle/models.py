@@ -145,7 +145,7 @@ def ref_tiny_gemma4():
     return hp, out
 
 
-# Named model shapes of BASELINE.json's configs.
+# Named model shapes of the benchmark's workloads.
 SHAPES = {
     # C1: tiny llama-style f32 model runnable on CPU.
     "c1": dict(arch="llama", n_layer=2, n_embd=256, n_head=4, n_head_kv=2, head_dim=64, n_ff=688,

@@ -1,18 +1,18 @@
 """Parity at the benchmark's own shapes: one decode pass of the forward at
 full width against the oracle, with the same synthetic KV on both sides.
 
-- C2 (configs[1]): 64 slots at the bench's LCG contexts U[128, 4096]
+- C2: 64 slots at the bench's LCG contexts U[128, 4096]
   (bench.py's draw order and seed), Llama-3-8B width, Q4_K_M, 1 layer.
-- C5 (configs[4]): 64 slots at contexts U[256, 8192], the 30B-A3B-shaped
+- C5: 64 slots at contexts U[256, 8192], the 30B-A3B-shaped
   qwen3moe width (128 experts of 768, top-8), Q4_K, 1 layer.
-- C4 (configs[3]): 32 slots at contexts U[1024, 16384], the Gemma-4-style
+- C4: 32 slots at contexts U[1024, 16384], the Gemma-4-style
   width (heads of 256, Q8_0, vocab 262144, softcap), a sliding layer (its
   1024-token window through each slot's ring) and a global layer.
 
 Every cell a pass reads holds the same random f16 K / V on both sides (the
 device pools are written through lgmlh_kv_store from the oracle's f16
 values, exact). Logits must be within 2e-3 max relative error of the
-oracle's and the greedy ids identical (BASELINE.json north star).
+oracle's and the greedy ids identical.
 
 The same passes in ggml's arithmetic (X quantized per block, what bench.py
 runs by default) cannot be held to 2e-3: ggml's arithmetic is not

@@ -1,4 +1,4 @@
-"""C3 (BASELINE.json configs[2]) against the oracle: sequences on a shared,
+"""C3 against the oracle: sequences on a shared,
 refcounted prefix, their suffixes prefilled in chunks mixed into the
 decode passes, at the C2 width (d 4096, 32 / 8 heads of 128, FFN 14336,
 vocab 128256, Q4_K_M) and 1 layer.

@@ -69,7 +69,7 @@ def test_hip_path_matches_llama_cpp_rows(arch):
 
 @pytest.mark.parametrize("arch", ["llama", "qwen3", "qwen3moe"])
 def test_gguf_loaded_models_match_llama_cpp_rows(tmp_path, arch):
-    """§8(f) row 3 end to end on the device: the tiny models written as gguf
+    """The loader end to end on the device: the tiny models written as gguf
     files with the reference's key-values and tensor names
     (test/test_qwen_moe.lua:65-200), read by runtime.load_gguf into a
     DeviceModel, meet the same llama.cpp rows."""

@@ -2,7 +2,7 @@
 
 Bit-exact: KV store (f32 -> f16 RNE), gather, block copy, dequantization,
 plan cells. Tolerance: attention and weight products within 2e-3 max
-relative error of the oracle's f64 result (BASELINE.json north star); the
+relative error of the oracle's f64 result; the
 kernels keep weights exact and split f32 activations into f16 hi + lo, so
 they also meet 1e-5 (products) and 1e-4 (attention). Batch invariance: a
 row alone and in a batch give the same bits.

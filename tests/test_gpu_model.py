@@ -1,6 +1,6 @@
 """End-to-end GPU parity of whole passes against the CPU oracle.
 
-C1 (BASELINE.json configs[0]): tiny llama-style f32 model, 4 slots with
+C1: tiny llama-style f32 model, 4 slots with
 prompts 17/64/129/300 prefilled in one ragged pass, then 32 greedy decode
 steps batched over the 4 slots. Greedy tokens must be identical; logits
 within 2e-3 max relative error. C2-shaped passes at reduced depth (2 layers,
@@ -79,7 +79,7 @@ def test_c2_shape_reduced_depth_ragged_decode(n_layer):
 def test_c2_full_depth_32_greedy_steps():
     """The full C2 model (32 layers, Q4_K_M, vocab 128256) on two short
     prompts, then 32 greedy steps batched over both: logits within 2e-3 of
-    the oracle and identical greedy streams (the north star's 32-step bar at
+    the oracle and identical greedy streams (the 32-step bar at
     the metric's own shape; the CPU oracle takes about 2 minutes here)."""
     hp, w = models.build("c2", seed=12, init="normal")
     prompts = [lcg_ints(3000, 8, 0, hp["n_vocab"]), lcg_ints(3001, 13, 0, hp["n_vocab"])]

@@ -1,4 +1,4 @@
-"""GPU parity of the routed-expert path (C5, BASELINE.json configs[4]) against
+"""GPU parity of the routed-expert path (C5) against
 the CPU oracle, through the C ABI.
 
 Routing (lgmlh_moe_route): ids bit-exact on the same logits (ties to the

@@ -1,4 +1,4 @@
-"""C3 (BASELINE.json configs[2]): prefix sharing through the engine.
+"""C3: prefix sharing through the engine.
 
 Requests that start with a prompt already in the pool attach its cached
 blocks (E:attach_blocks, lua/lgml/engine.lua:2038-2077): full blocks are
